@@ -313,12 +313,15 @@ struct CheckParams {
 // check_if_window_is_flat + average_and_redistribute_window + reset_counts +
 // the ln f schedule (rewl_simulation.hpp:458-470, 361-454, 541-598;
 // rewl_histograms.hpp:83-95, 115-152).
-__global__ void __launch_bounds__(kLanes) k_check(KArgs a, CheckParams cp, int32_t* flat_out) {
+__global__ void __launch_bounds__(kLanes) k_check(KArgs a, CheckParams cp, int32_t* flat_out, int32_t* done_out) {
     const int wi = blockIdx.x;
     if (wi >= a.num_windows) return;
     const int lane = threadIdx.x;
     if (!a.win_active[wi]) {   // a retired system: state kept as it was
-        if (lane == 0) flat_out[wi] = 0;
+        if (lane == 0) {
+            flat_out[wi] = 0;
+            done_out[wi] = a.win_done[wi];
+        }
         return;
     }
     const DevWindow W = a.win[wi];
@@ -420,6 +423,7 @@ __global__ void __launch_bounds__(kLanes) k_check(KArgs a, CheckParams cp, int32
         }
         a.win_sweeps[wi] = sw;
         flat_out[wi] = flat ? 1 : 0;
+        done_out[wi] = a.win_done[wi];
     }
 }
 

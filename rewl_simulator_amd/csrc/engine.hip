@@ -146,7 +146,7 @@ struct rewl_ctx {
     int tuned_nprod = 2;
     DevBuf<int32_t> d_tuned_groups[2][5];
     std::vector<int32_t> pairs_even, pairs_odd;
-    DevBuf<int32_t> d_pairs_even, d_pairs_odd, d_flat;
+    DevBuf<int32_t> d_pairs_even, d_pairs_odd;
 
     DevBuf<DevSystem> d_sys;
     DevBuf<DevWindow> d_win;
@@ -166,6 +166,12 @@ struct rewl_ctx {
     DevBuf<BoundEntry> d_bound_tab;
     DevBuf<double> d_obs;       // observable sums (observables on)
     DevBuf<double> d_stage;     // rewl_set_logdos: one walker's ln g, copied linearly, then scattered
+    // Pinned host memory that kernels write query results into (fetch), and
+    // the flat / done flags of rewl_check: [2 * windows]
+    std::mutex fetch_mu;
+    void* h_fetch = nullptr;
+    size_t h_fetch_bytes = 0;
+    int32_t* h_check = nullptr;
     DevBuf<uint32_t> d_obs_tot; // updates so far per (bin, walker) (observables with correlators)
     DevBuf<uint32_t> d_dens;    // AT sigma-tau density counts [(hist index) * 1024 + cell] (densities on)
     int nobs = 0;
@@ -198,7 +204,7 @@ void destroy_ctx(rewl_ctx* c) {
     c->ev_sweep.clear();
     for (auto* b : {&c->d_w_window, &c->d_w_local, &c->d_w_flavor, &c->d_err, &c->d_win_oot, &c->d_win_done,
                     &c->d_win_active,
-                    &c->d_pairs_even, &c->d_pairs_odd, &c->d_flat})
+                    &c->d_pairs_even, &c->d_pairs_odd})
         b->release();
     for (auto& b : c->d_class_groups) b.release();
     for (auto& row : c->d_tuned_groups)
@@ -208,6 +214,8 @@ void destroy_ctx(rewl_ctx* c) {
     c->d_w_cursor.release(); c->d_lat.release(); c->d_visits.release(); c->d_ring.release(); c->d_ring_filled.release();
     c->d_exclude.release(); c->d_lng.release(); c->d_cnt.release(); c->d_exch.release(); c->d_bound_tab.release(); c->d_obs.release(); c->d_obs_tot.release(); c->d_dens.release(); c->d_stage.release();
     c->d_sys.release(); c->d_win.release(); c->d_grp.release();
+    if (c->h_fetch) (void)hipHostFree(c->h_fetch);
+    if (c->h_check) (void)hipHostFree(c->h_check);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -227,6 +235,62 @@ int overwrite(DevBuf<T>& b, const std::vector<T>& v, hipStream_t s) {
     return REWL_OK;
 }
 
+// Query results.  A walker's column of a histogram is one element (or `width`)
+// per row of 64 lanes; copied by hipMemcpy2D every element is a copy of its
+// own (1.6 ms for the 236 doubles of an L = 64 window, 0.45 ms for 64 rows of
+// spins), and even one value copied to pageable memory costs 29 us.  A gather
+// kernel that writes into pinned memory of the context and one stream
+// synchronisation take about 15 us for any of them.
+template <typename T>
+__global__ void k_gather(T* dst, const T* src, int64_t stride, int rows, int width) {
+    const int n = rows * width;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        dst[i] = src[(int64_t)(i / width) * stride + i % width];
+}
+
+// Room for `bytes` in the pinned buffer (fetch_mu held).
+int reserve_fetch(rewl_ctx* c, size_t bytes) {
+    if (bytes <= c->h_fetch_bytes) return REWL_OK;
+    if (c->h_fetch) (void)hipHostFree(c->h_fetch);
+    c->h_fetch = nullptr;
+    c->h_fetch_bytes = 0;
+    const size_t want = std::max<size_t>(bytes, 16384);
+    HIP_TRY(hipHostMalloc(&c->h_fetch, want, hipHostMallocDefault));
+    c->h_fetch_bytes = want;
+    return REWL_OK;
+}
+
+// out[r * width + i] = src[r * stride + i] for r < rows, i < width, after all
+// work queued on the context's stream.
+template <typename T>
+int fetch(rewl_ctx* c, const T* src, int64_t stride, int rows, int width, T* out) {
+    std::lock_guard<std::mutex> lock(c->fetch_mu);
+    const size_t n = (size_t)rows * (size_t)width;
+    int rc;
+    if ((rc = reserve_fetch(c, n * sizeof(T)))) return rc;
+    const unsigned grid = (unsigned)std::min<size_t>(256, (n + 255) / 256);
+    hipLaunchKernelGGL(k_gather<T>, dim3(grid), dim3(256), 0, c->stream, static_cast<T*>(c->h_fetch), src, stride, rows,
+                       width);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    std::memcpy(out, c->h_fetch, n * sizeof(T));
+    return REWL_OK;
+}
+
+// The changing part of a window's record, written to pinned memory.
+struct WindowState {
+    double lnf;
+    int64_t iteration, sweeps;
+    int32_t done, one_over_t;
+};
+__global__ void k_window_state(KArgs a, int wi, WindowState* out) {
+    out->lnf = a.win_lnf[wi];
+    out->iteration = a.win_iter[wi];
+    out->sweeps = a.win_sweeps[wi];
+    out->done = a.win_done[wi];
+    out->one_over_t = a.win_oot[wi];
+}
+
 int resolve_sweep_events(rewl_ctx* c) {
     for (auto& e : c->ev_sweep) {
         HIP_TRY(hipEventSynchronize(e.second));
@@ -243,8 +307,8 @@ int resolve_sweep_events(rewl_ctx* c) {
 
 int check_err_flag(rewl_ctx* c) {
     int32_t e = 0;
-    HIP_TRY(hipMemcpyAsync(&e, c->d_err.p, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    int rc;
+    if ((rc = fetch(c, c->d_err.p, 1, 1, 1, &e))) return rc;
     if (e & 1) return fail(REWL_ERR_REPLAY, "replay stream exhausted");
     if (e & 2) return fail(REWL_ERR_RANGE, "a walker could not be brought into its window");
     return REWL_OK;
@@ -252,8 +316,8 @@ int check_err_flag(rewl_ctx* c) {
 
 int clear_err_bits(rewl_ctx* c, int32_t bits) {
     int32_t e = 0;
-    HIP_TRY(hipMemcpyAsync(&e, c->d_err.p, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    int rc;
+    if ((rc = fetch(c, c->d_err.p, 1, 1, 1, &e))) return rc;
     if (!(e & bits)) return REWL_OK;
     e &= ~bits;
     HIP_TRY(hipMemcpyAsync(c->d_err.p, &e, sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
@@ -801,13 +865,14 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         for (int i = 0; i < 5; ++i) c->tuned_groups_all[m][i] = c->tuned_groups[m][i];
     c->pairs_even_all = c->pairs_even;
     c->pairs_odd_all = c->pairs_odd;
-    if ((rc = upload(c->d_flat, zeros32, c->stream))) return bail(rc);
     if ((rc = upload(c->d_w_flavor, flav, c->stream))) return bail(rc);
     if ((rc = upload(c->d_w_E, E0, c->stream))) return bail(rc);
     if ((rc = upload(c->d_w_cursor, cur0, c->stream))) return bail(rc);
     if ((rc = upload(c->d_err, std::vector<int32_t>(1, 0), c->stream))) return bail(rc);
     if ((rc = upload(c->d_exch, std::vector<unsigned long long>(1, 0ull), c->stream))) return bail(rc);
     c->done_host.assign(nwin, 0);
+    if (hipHostMalloc((void**)&c->h_check, 2 * nwin * sizeof(int32_t), hipHostMallocDefault) != hipSuccess)
+        return bail(fail(REWL_ERR_DEVICE, "hipHostMalloc failed"));
 
     if (c->d_lat.alloc(c->lat_total) != hipSuccess || c->d_lng.alloc(c->hist_total) != hipSuccess ||
         c->d_cnt.alloc(c->hist_total) != hipSuccess || c->d_visits.alloc(c->hist_total) != hipSuccess)
@@ -1052,13 +1117,14 @@ int rewl_check(rewl_ctx* c) {
     cp.lnf_final = c->p.lnf_final;
     cp.pending_sweeps = c->pending_sweeps;
     const int nwin = (int)c->win.size();
-    hipLaunchKernelGGL(k_check, dim3((unsigned)nwin), dim3(kLanes), 0, c->stream, c->args, cp, c->d_flat.p);
+    // the kernel writes each window's flat and done flags to pinned memory
+    int32_t* const flat = c->h_check;
+    int32_t* const done = c->h_check + nwin;
+    hipLaunchKernelGGL(k_check, dim3((unsigned)nwin), dim3(kLanes), 0, c->stream, c->args, cp, flat, done);
     HIP_TRY(hipGetLastError());
     c->pending_sweeps = 0;
-    std::vector<int32_t> flat((size_t)nwin);
-    HIP_TRY(hipMemcpyAsync(c->done_host.data(), c->d_win_done.p, (size_t)nwin * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(flat.data(), c->d_flat.p, (size_t)nwin * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
+    std::copy(done, done + nwin, c->done_host.begin());
     int all = 1;
     for (int k = 0; k < nwin; ++k) {
         all &= c->done_host[k] ? 1 : 0;
@@ -1183,17 +1249,20 @@ int rewl_get_window_info(rewl_ctx* c, int32_t wi, rewl_window_info* o) {
     o->first_walker = w.first_walker;
     o->num_bins = w.nbins;
     o->e_min = w.emin; o->e_max = w.emax; o->bin_size = w.bs;
-    int32_t done = 0, oot = 0;
-    int64_t sweeps = 0;
-    HIP_TRY(hipMemcpyAsync(&o->lnf, c->d_win_lnf.p + wi, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(&o->iteration, c->d_win_iter.p + wi, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(&sweeps, c->d_win_sweeps.p + wi, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(&done, c->d_win_done.p + wi, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(&oot, c->d_win_oot.p + wi, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
+    std::lock_guard<std::mutex> lock(c->fetch_mu);
+    int rc;
+    if ((rc = reserve_fetch(c, sizeof(WindowState)))) return rc;
+    hipLaunchKernelGGL(k_window_state, dim3(1), dim3(1), 0, c->stream, c->args, (int)wi,
+                       static_cast<WindowState*>(c->h_fetch));
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(c->stream));
-    o->sweeps_in_iteration = sweeps + c->pending_sweeps;
-    o->done = done;
-    o->one_over_t = oot;
+    WindowState s;
+    std::memcpy(&s, c->h_fetch, sizeof(s));
+    o->lnf = s.lnf;
+    o->iteration = s.iteration;
+    o->sweeps_in_iteration = s.sweeps + c->pending_sweeps;
+    o->done = s.done;
+    o->one_over_t = s.one_over_t;
     return REWL_OK;
 }
 
@@ -1202,8 +1271,7 @@ int rewl_get_stats(rewl_ctx* c, rewl_stats* o) {
     int rc;
     if ((rc = resolve_sweep_events(c))) return rc;
     unsigned long long acc = 0;
-    HIP_TRY(hipMemcpyAsync(&acc, c->d_exch.p, sizeof(acc), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    if ((rc = fetch(c, c->d_exch.p, 1, 1, 1, &acc))) return rc;
     c->stats.exchanges_accepted = acc;
     *o = c->stats;
     return REWL_OK;
@@ -1215,30 +1283,21 @@ int rewl_get_logdos(rewl_ctx* c, int32_t g, double* out, int32_t n) {
     if (!walker_ok(c, g) || !out) return fail(REWL_ERR_INVALID, "bad walker");
     const int nb = c->win[c->w_window[g]].nbins;
     if (n < nb) return fail(REWL_ERR_INVALID, "output buffer too small");
-    HIP_TRY(hipMemcpy2DAsync(out, sizeof(double), c->d_lng.p + c->w_hist[g], kLanes * sizeof(double), sizeof(double),
-                             (size_t)nb, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REWL_OK;
+    return fetch(c, c->d_lng.p + c->w_hist[g], kLanes, nb, 1, out);
 }
 
 int rewl_get_counts(rewl_ctx* c, int32_t g, uint32_t* out, int32_t n) {
     if (!walker_ok(c, g) || !out) return fail(REWL_ERR_INVALID, "bad walker");
     const int nb = c->win[c->w_window[g]].nbins;
     if (n < nb) return fail(REWL_ERR_INVALID, "output buffer too small");
-    HIP_TRY(hipMemcpy2DAsync(out, sizeof(uint32_t), c->d_cnt.p + c->w_hist[g], kLanes * sizeof(uint32_t),
-                             sizeof(uint32_t), (size_t)nb, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REWL_OK;
+    return fetch(c, c->d_cnt.p + c->w_hist[g], kLanes, nb, 1, out);
 }
 
 int rewl_get_visits(rewl_ctx* c, int32_t g, uint64_t* out, int32_t n) {
     if (!walker_ok(c, g) || !out) return fail(REWL_ERR_INVALID, "bad walker");
     const int nb = c->win[c->w_window[g]].nbins;
     if (n < nb) return fail(REWL_ERR_INVALID, "output buffer too small");
-    HIP_TRY(hipMemcpy2DAsync(out, sizeof(uint64_t), c->d_visits.p + c->w_hist[g], kLanes * sizeof(uint64_t),
-                             sizeof(uint64_t), (size_t)nb, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REWL_OK;
+    return fetch(c, c->d_visits.p + c->w_hist[g], kLanes, nb, 1, out);
 }
 
 int rewl_get_observables(rewl_ctx* c, int32_t g, double* sums, int32_t n, int32_t nobs) {
@@ -1251,11 +1310,7 @@ int rewl_get_observables(rewl_ctx* c, int32_t g, double* sums, int32_t n, int32_
     if (nobs != want) return fail(REWL_ERR_INVALID, "nobs does not match the walker's model");
     const int nb = c->win[c->w_window[g]].nbins;
     if (n < nb) return fail(REWL_ERR_INVALID, "output buffer too small");
-    HIP_TRY(hipMemcpy2DAsync(sums, (size_t)nobs * sizeof(double), c->d_obs.p + c->w_hist[g] * c->nobs,
-                             (size_t)kLanes * c->nobs * sizeof(double), (size_t)nobs * sizeof(double), (size_t)nb,
-                             hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REWL_OK;
+    return fetch(c, c->d_obs.p + c->w_hist[g] * c->nobs, (int64_t)kLanes * c->nobs, nb, nobs, sums);
 }
 
 int rewl_get_densities(rewl_ctx* c, int32_t g, uint32_t* out, int32_t n) {
@@ -1276,9 +1331,8 @@ int rewl_get_spins(rewl_ctx* c, int32_t g, int8_t* out, int32_t n) {
     if (n < S.ndof) return fail(REWL_ERR_INVALID, "output buffer too small");
     const int planes = model_info(S.d.model).planes, L = S.d.L;
     std::vector<uint64_t> words((size_t)planes * L);
-    HIP_TRY(hipMemcpy2DAsync(words.data(), sizeof(uint64_t), c->d_lat.p + c->w_lat[g], kLanes * sizeof(uint64_t),
-                             sizeof(uint64_t), words.size(), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    int rc;
+    if ((rc = fetch(c, c->d_lat.p + c->w_lat[g], kLanes, (int)words.size(), 1, words.data()))) return rc;
     for (int i = 0; i < S.N; ++i) {
         const int x = i % L, y = i / L;
         for (int q = 0; q < planes; ++q) {
@@ -1291,23 +1345,17 @@ int rewl_get_spins(rewl_ctx* c, int32_t g, int8_t* out, int32_t n) {
 
 int rewl_get_energy(rewl_ctx* c, int32_t g, double* e) {
     if (!walker_ok(c, g) || !e) return fail(REWL_ERR_INVALID, "bad walker");
-    HIP_TRY(hipMemcpyAsync(e, c->d_w_E.p + g, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REWL_OK;
+    return fetch(c, c->d_w_E.p + g, 1, 1, 1, e);
 }
 
 int rewl_get_flavor(rewl_ctx* c, int32_t g, int32_t* f) {
     if (!walker_ok(c, g) || !f) return fail(REWL_ERR_INVALID, "bad walker");
-    HIP_TRY(hipMemcpyAsync(f, c->d_w_flavor.p + g, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REWL_OK;
+    return fetch(c, c->d_w_flavor.p + g, 1, 1, 1, f);
 }
 
 int rewl_get_rng_cursor(rewl_ctx* c, int32_t g, uint64_t* cur) {
     if (!walker_ok(c, g) || !cur) return fail(REWL_ERR_INVALID, "bad walker");
-    HIP_TRY(hipMemcpyAsync(cur, c->d_w_cursor.p + g, sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REWL_OK;
+    return fetch(c, c->d_w_cursor.p + g, 1, 1, 1, cur);
 }
 
 // One walker's ln g column ([bin][lane] layout) from a linear staging copy.
