@@ -165,12 +165,14 @@ typedef struct rewl_params {
                                     1 = equal weights 1/R, the alternative left in
                                     rewl_simulation.hpp:401 (unbiased when replicas
                                     also exchange with other windows)               */
-    int32_t sweep_kernel;        /* Philox integer path: 0 = auto (3 for L in
-                                    {16,24,32,48,64}, else 1); 1 = row kernel;
-                                    2 = row-unrolled; 3 = row-unrolled with the
-                                    next slot computed for both outcomes; 4 = that
-                                    and the next ln g read ahead (2-4 are an error
-                                    for other L or producers < 0)                  */
+    int32_t sweep_kernel;        /* Philox integer path: 0 = auto (sixteen lanes per
+                                    walker in contexts of up to 4096 walkers, else 3
+                                    for L in {16,24,32,48,64}, else 1); 1 = row
+                                    kernel; 2 = row-unrolled; 3 = row-unrolled with
+                                    the next slot computed for both outcomes; 4 =
+                                    that and the next ln g read ahead (2-4 are an
+                                    error for other L or producers < 0).  Every
+                                    kernel runs the same chain                      */
     int32_t observables;         /* 1: per-bin observable sums of every update (each
                                     attempt and each post-exchange increment) at the
                                     walker's current bin: |m|, m^2, m^4 (Ising,

@@ -6,6 +6,7 @@
 import os
 import subprocess
 import sys
+import tempfile
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -21,7 +22,6 @@ HIP_FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # the row-unrolled sweep kernel unrolls L attempts (with their rare exact
@@ -32,14 +32,27 @@ HIP_FLAGS = [
 ]
 
 
+# One object per translation unit, compiled side by side.
+ENGINE_SOURCES = ["engine.hip", "tuned_kernels.hip"]
+
+
 def build_engine(verbose=False):
-    src = os.path.join(CSRC, "engine.hip")
-    tmp = ENGINE_SO + ".tmp"
-    cmd = [HIPCC, *HIP_FLAGS, "-I", os.path.join(ROOT, "include"), src, "-o", tmp]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
-    os.replace(tmp, ENGINE_SO)
+    with tempfile.TemporaryDirectory() as tmp:
+        jobs, objs = [], []
+        for name in ENGINE_SOURCES:
+            obj = os.path.join(tmp, name + ".o")
+            cmd = [HIPCC, *HIP_FLAGS, "-c", "-I", os.path.join(ROOT, "include"), os.path.join(CSRC, name), "-o", obj]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            jobs.append((cmd, subprocess.Popen(cmd)))
+            objs.append(obj)
+        codes = [(cmd, p.wait()) for cmd, p in jobs]
+        for cmd, rc in codes:
+            if rc:
+                raise subprocess.CalledProcessError(rc, cmd)
+        out = ENGINE_SO + ".tmp"
+        subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", out], check=True)
+        os.replace(out, ENGINE_SO)
     return ENGINE_SO
 
 

@@ -25,7 +25,13 @@
 #include "sweep_fast.hpp"
 #include "sweep_field.hpp"
 #include "sweep_tuned.hpp"
+#include "sweep_tree.hpp"
 #include "anneal.hpp"
+
+namespace rewl {
+// tuned_kernels.hip
+const void* tuned_kernel(int model, int L, bool simple, int spec, int obs);
+}  // namespace rewl
 
 static_assert(REWL_ISING2D == 0 && REWL_ASHKIN_TELLER2D == 1, "the C ABI's model index is Model<M>'s M");
 
@@ -108,11 +114,35 @@ std::vector<HostWindow> make_windows(const rewl_system_desc& d) {
 
 bool integral(double v) { return std::isfinite(v) && std::floor(v) == v && std::fabs(v) < 1e9; }
 
+// k_sweep_tree takes contexts of at most this many walkers: with 4096 its
+// workgroups (sixteen walkers, one per CU) fill the chip, and a second round of
+// them doubles its time per attempt while the kernels with one lane per walker
+// still have room.  Measured, cycles per attempt, tree against lane: L = 64
+// Ising 104 / 161 at 512 walkers, 115 / 159 at 2048, 137 / 159 at 4096, 273 /
+// 159 at 5120; L = 32 Ashkin-Teller 128 / 198, 137 / 197, 155 / 197, 231 / 197.
+// Sizes without an unrolled-row kernel have the row kernel to compare with
+// (480-540 cycles): 215 at 8192, 389 at 12288.
+constexpr int kTreeMaxWalkers = 4096, kTreeMaxWalkersRow = 12288;
+
 constexpr int kTunedL[5] = {16, 24, 32, 48, 64};
 int tuned_index(int L) {
     for (int i = 0; i < 5; ++i)
         if (kTunedL[i] == L) return i;
     return -1;
+}
+
+// Whether the reference's range test on a system's integer energies is plainly
+// min <= E < max: E = -1 collides with E = 0 in its +0.5 truncation, which
+// matters only if E = -1 is reachable and a window bound is 0.
+bool simple_range(const HostSystem& S, const std::vector<HostWindow>& win) {
+    const ModelInfo mi = model_info(S.d.model);
+    const long long g = mi.energy_step(S.twoJ, S.twoK);
+    const long long e0 = mi.ground_energy(S.N, S.twoJ, S.twoK);
+    bool zero_bound = false;
+    for (int k = 0; k < S.d.num_windows; ++k)
+        zero_bound = zero_bound || win[S.first_window + k].emin == 0.0 || win[S.first_window + k].emax == 0.0;
+    const bool m1_reachable = g == 0 ? (e0 == -1) : (((-1 - e0) % g) == 0);
+    return !(zero_bound && m1_reachable);
 }
 
 }  // namespace
@@ -145,6 +175,12 @@ struct rewl_ctx {
     int tuned_guard[2][5] = {};                          // guard bins each side: max |Delta E| / bin size
     int tuned_nprod = 2;
     DevBuf<int32_t> d_tuned_groups[2][5];
+    // sixteen-lanes-a-walker kernel (sweep_tree.hpp): group lists per model
+    std::vector<int32_t> tree_groups[2], tree_groups_all[2];
+    DevBuf<int32_t> d_tree_groups[2];
+    DevBuf<TreeScale> d_tree_scale;                      // per system
+    size_t tree_lds_bytes[2] = {0, 0};                   // the largest group's LDS
+    int tree_nw = 1;                                     // walker wavefronts per workgroup
     std::vector<int32_t> pairs_even, pairs_odd;
     DevBuf<int32_t> d_pairs_even, d_pairs_odd;
 
@@ -209,6 +245,8 @@ void destroy_ctx(rewl_ctx* c) {
     for (auto& b : c->d_class_groups) b.release();
     for (auto& row : c->d_tuned_groups)
         for (auto& b : row) b.release();
+    for (auto& b : c->d_tree_groups) b.release();
+    c->d_tree_scale.release();
     c->d_w_hist.release(); c->d_w_lat.release(); c->d_win_iter.release(); c->d_win_sweeps.release();
     c->d_w_E.release(); c->d_win_lnf.release(); c->d_fields.release();
     c->d_w_cursor.release(); c->d_lat.release(); c->d_visits.release(); c->d_ring.release(); c->d_ring_filled.release();
@@ -430,14 +468,9 @@ int launch_sweep_tuned(rewl_ctx* c, int li, int nsweeps) {
     // sweep_kernel 2: no speculation, 3 (and auto): next slot for both outcomes,
     // 4: that and the next ln g read ahead
     const int sk = c->p.sweep_kernel;
-    void* kern;
-    if (sk == 2) kern = simple ? (void*)k_sweep_tuned<MODEL, L, true, 0> : (void*)k_sweep_tuned<MODEL, L, false, 0>;
-    else if (sk == 4) kern = simple ? (void*)k_sweep_tuned<MODEL, L, true, 2> : (void*)k_sweep_tuned<MODEL, L, false, 2>;
-    else if (c->p.observables == 2)
-        kern = simple ? (void*)k_sweep_tuned<MODEL, L, true, 1, 2> : (void*)k_sweep_tuned<MODEL, L, false, 1, 2>;
-    else if (c->p.observables)
-        kern = simple ? (void*)k_sweep_tuned<MODEL, L, true, 1, 1> : (void*)k_sweep_tuned<MODEL, L, false, 1, 1>;
-    else kern = simple ? (void*)k_sweep_tuned<MODEL, L, true, 1> : (void*)k_sweep_tuned<MODEL, L, false, 1>;
+    const int spec = sk == 2 ? 0 : sk == 4 ? 2 : 1;
+    const void* kern = tuned_kernel(MODEL, L, simple, spec, spec == 1 ? c->p.observables : 0);
+    if (!kern) return fail(REWL_ERR_INVALID, "internal: no row-unrolled kernel of this form");
     HIP_TRY(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     KArgs args = c->args;
     const int32_t* gl = c->d_tuned_groups[MODEL][li].p;
@@ -445,6 +478,24 @@ int launch_sweep_tuned(rewl_ctx* c, int li, int nsweeps) {
     int guard_arg = guard;
     void* kargs[] = {&args, (void*)&gl, (void*)&ng, (void*)&nsweeps, (void*)&base, (void*)&guard_arg};
     HIP_TRY(hipLaunchKernel((const void*)kern, dim3((unsigned)ng), dim3(kLanes * (1 + np)), kargs, lds, c->stream));
+    HIP_TRY(hipGetLastError());
+    return REWL_OK;
+}
+
+// Producer wavefronts of a k_sweep_tree workgroup: with one or two walker
+// wavefronts each of the four has a SIMD of its own.
+int tree_producers(int nw) { return nw <= 2 ? 2 : 4; }
+
+template <int MODEL>
+int launch_sweep_tree(rewl_ctx* c, int nsweeps) {
+    const int ng = (int)c->tree_groups[MODEL].size();
+    if (ng == 0) return REWL_OK;
+    const size_t lds = c->tree_lds_bytes[MODEL];
+    const int nw = c->tree_nw;
+    HIP_TRY(hipFuncSetAttribute((const void*)k_sweep_tree<MODEL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_sweep_tree<MODEL>, dim3((unsigned)ng), dim3((unsigned)(kLanes * (nw + tree_producers(nw)))), lds,
+                       c->stream, c->args, (const TreeScale*)c->d_tree_scale.p, (const int32_t*)c->d_tree_groups[MODEL].p,
+                       ng, nsweeps, c->sweep_index, nw);
     HIP_TRY(hipGetLastError());
     return REWL_OK;
 }
@@ -506,10 +557,43 @@ int launch_sweeps(rewl_ctx* c, int nsweeps) {
     if ((rc = launch_sweep_class<1, true>(c, 3, nsweeps))) return rc;
     if ((rc = launch_tuned_all<0>(c, nsweeps))) return rc;
     if ((rc = launch_tuned_all<1>(c, nsweeps))) return rc;
+    if ((rc = launch_sweep_tree<0>(c, nsweeps))) return rc;
+    if ((rc = launch_sweep_tree<1>(c, nsweeps))) return rc;
     HIP_TRY(hipEventRecord(e1, c->stream));
     c->ev_sweep.emplace_back(e0, e1);
     if (c->ev_sweep.size() > 256) return resolve_sweep_events(c);
     return REWL_OK;
+}
+
+// Byte scale of a system's states and energy changes in k_sweep_tree with `nw`
+// walker wavefronts per workgroup, and whether that kernel takes the system:
+// the state is energy x pitch / bin, stored energy changes are signed bytes
+// and their weight too.
+bool tree_scale(const rewl_system_desc& d, int twoJ, int twoK, int nw, TreeScale* out) {
+    const bool kq = model_info(d.model).product_coupling;
+    const long long bin = (long long)d.bin_size;
+    if (bin < 1 || bin > 256) return false;
+    const long long aJ = std::abs((long long)twoJ), aK = kq ? std::abs((long long)twoK) : 0;
+    if (aJ > 1000000 || aK > 1000000) return false;
+    const long long g = std::gcd(2 * aJ, 2 * aK);   // energy changes: twoJ (4 - 2 k) + twoK (4 - 2 q)
+    if (g == 0) return false;
+    TreeScale t{};
+    const long long pitch = std::max<long long>(8 * kTreePerWave * nw, bin);
+    const long long unit = pitch / bin * g;
+    long long m = 1;
+    while (unit / m > 127 && unit % (2 * m) == 0) m *= 2;
+    if (unit / m > 127) return false;
+    const long long most = kq ? 63 : 127;
+    if (4 * aJ / g * m > most || 4 * aK / g * m > most) return false;
+    // four proposals ahead of a state inside the window
+    const long long reach = 4 * (4 * aJ + 4 * aK);
+    t.pitch = (int)pitch;
+    t.g = (int)g;
+    t.m = (int)m;
+    t.w = (int)(unit / m);
+    t.guard = (int)((reach + bin - 1) / bin) + 1;
+    *out = t;
+    return true;
 }
 
 int max_ndof(const rewl_ctx* c) {
@@ -628,6 +712,43 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(REWL_ERR_DEVICE, "hipStreamCreate failed"));
 
+    // ---- systems swept with sixteen lanes a walker -------------------------------
+    // When the caller asks for no particular kernel or launch shape and the
+    // context has few enough walkers (kTreeMaxWalkers).  One, two or four
+    // walker wavefronts (4, 8, 16 walkers) per workgroup, so that the
+    // workgroups of a small context spread over the CUs (104 cycles an attempt
+    // alone on a CU, 115 with a second walker wavefront, 137 with four), as far
+    // as the LDS of the widest window allows.
+    std::vector<uint8_t> tree_sys(c->sys.size(), 0);
+    std::vector<TreeScale> tree_scales(c->sys.size());
+    {
+        const bool shape_free = P.rng_mode == REWL_RNG_PHILOX && P.observables == 0 && P.sweep_kernel == 0 &&
+                                P.producers == 0 && P.walkers_per_group == 0;
+        c->tree_nw = W <= 1024 ? 1 : W <= 2048 ? 2 : 4;
+        auto fits = [&](const HostSystem& S, int nw, TreeScale* t) {
+            if (!tree_scale(S.d, S.twoJ, S.twoK, nw, t)) return false;
+            int nb = 1;
+            for (int k = 0; k < S.d.num_windows; ++k) nb = std::max(nb, c->win[S.first_window + k].nbins);
+            const long long bytes = (long long)(nb + 2 * t->guard) * t->pitch * 2;
+            if (bytes > 4LL * c->lds_max) return false;   // keeps the sums below in range
+            return (size_t)tree_lds(model_info(S.d.model).planes, S.d.L, nb, nw, t->pitch, t->guard).total <=
+                   (size_t)c->lds_max;
+        };
+        for (size_t si = 0; shape_free && si < c->sys.size(); ++si) {
+            const HostSystem& S = c->sys[si];
+            if (W > (tuned_index(S.d.L) >= 0 ? kTreeMaxWalkers : kTreeMaxWalkersRow)) continue;
+            if (!S.intpath || S.d.L < kTreeMinL || !simple_range(S, c->win)) continue;
+            TreeScale t;
+            int nw = c->tree_nw;
+            while (nw >= 1 && !fits(S, nw, &t)) nw /= 2;
+            if (nw < 1) continue;
+            c->tree_nw = nw;
+            tree_sys[si] = 1;
+        }
+        for (size_t si = 0; si < c->sys.size(); ++si)
+            if (tree_sys[si] && !fits(c->sys[si], c->tree_nw, &tree_scales[si])) tree_sys[si] = 0;
+    }
+
     // ---- wavefront groups -----------------------------------------------------
     c->w_group.assign(W, 0);
     c->w_lane.assign(W, 0);
@@ -653,13 +774,14 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         const int li = tuned_index(S.d.L);
         // observables (without densities) also run on the row-unrolled kernel, in its default form
         const bool tuned_obs = P.observables >= 1 && !P.densities && P.sweep_kernel != 2 && P.sweep_kernel != 4;
-        const bool tuned = S.intpath && P.rng_mode == REWL_RNG_PHILOX && (!obs || tuned_obs) && P.producers >= 0 &&
+        const bool tree = tree_sys[(size_t)si] != 0;
+        const bool tuned = !tree && S.intpath && P.rng_mode == REWL_RNG_PHILOX && (!obs || tuned_obs) && P.producers >= 0 &&
                            li >= 0 && P.sweep_kernel != 1;
         if (P.sweep_kernel >= 2 && !tuned)
             return bail(fail(REWL_ERR_INVALID, "the row-unrolled kernel needs the Philox integer path, producers >= 0 "
                                                "and L in {16, 24, 32, 48, 64}; with observables, sweep_kernel 0 or 3 "
                                                "and no densities"));
-        int wpg = kLanes;
+        int wpg = tree ? c->tree_nw * kTreePerWave : kLanes;
         // guard bins: |Delta E| <= 4 (2J) (+ 4 (2K)) on the integer path
         int guard = 0;
         if (tuned) {
@@ -673,7 +795,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
                                                  (size_t)tuned_ring_stride(S.d.L) +
                                                  (size_t)maxbins * tuned_obs_bytes(S.d.model, P.observables))));
         }
-        else if (fast)
+        else if (fast && !tree)
             wpg = std::min(kLanes, (int)((size_t)c->lds_max /
                                          ((size_t)(maxbins + 1) * 12 + (c->nprod ? 8 * (size_t)S.d.L : 0))));
         else if (field_fast) {
@@ -686,23 +808,15 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         }
         if (P.walkers_per_group > 0) wpg = std::min(wpg, (int)P.walkers_per_group);
         if (wpg < 1) return bail(fail(REWL_ERR_INVALID, "window too wide for LDS: " + std::to_string(maxbins) + " bins"));
-        {
-            // E = -1 collides with E = 0 in the reference's +0.5 range test; it
-            // matters only if E = -1 is reachable and a window bound is 0.
-            const ModelInfo mi = model_info(S.d.model);
-            const long long g = mi.energy_step(S.twoJ, S.twoK);
-            const long long e0 = mi.ground_energy(S.N, S.twoJ, S.twoK);
-            bool zero_bound = false;
-            for (int k = 0; k < S.d.num_windows; ++k)
-                zero_bound = zero_bound || c->win[S.first_window + k].emin == 0.0 || c->win[S.first_window + k].emax == 0.0;
-            const bool m1_reachable = g == 0 ? (e0 == -1) : (((-1 - e0) % g) == 0);
+        if (!tree) {
+            const bool simple = simple_range(S, c->win);
             if (tuned) {
-                if (zero_bound && m1_reachable) c->tuned_simple[S.d.model][li] = false;
+                if (!simple) c->tuned_simple[S.d.model][li] = false;
                 c->tuned_maxlanes[S.d.model][li] = std::max(c->tuned_maxlanes[S.d.model][li], wpg);
                 c->tuned_guard[S.d.model][li] = std::max(c->tuned_guard[S.d.model][li], guard);
             } else {
                 const int cls = S.d.model * 2 + (S.intpath ? 1 : 0);
-                if (zero_bound && m1_reachable) c->class_simple[cls] = false;
+                if (!simple) c->class_simple[cls] = false;
                 c->class_maxlanes[cls] = std::max(c->class_maxlanes[cls], wpg);
                 c->class_maxL[cls] = std::max(c->class_maxL[cls], S.d.L);
                 if (field_fast) c->class_field[cls] = true;
@@ -728,7 +842,13 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
                 c->w_hist[g] = G.hist_base + j;
                 c->w_lat[g] = G.lat_base + j;
             }
-            if (tuned) {
+            if (tree) {
+                c->tree_groups[S.d.model].push_back(gid);
+                const TreeScale& t = tree_scales[(size_t)si];
+                c->tree_lds_bytes[S.d.model] =
+                    std::max(c->tree_lds_bytes[S.d.model],
+                             (size_t)tree_lds(planes, S.d.L, nb, c->tree_nw, t.pitch, t.guard).total);
+            } else if (tuned) {
                 c->tuned_groups[S.d.model][li].push_back(gid);
                 c->tuned_maxbins[S.d.model][li] = std::max(c->tuned_maxbins[S.d.model][li], nb);
             } else {
@@ -832,6 +952,13 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         std::stable_sort(c->class_groups[cls].begin(), c->class_groups[cls].end(), [&](int32_t x, int32_t y) {
             return c->sys[(size_t)c->groups[(size_t)x].sys].ndof > c->sys[(size_t)c->groups[(size_t)y].sys].ndof;
         });
+    for (auto& list : c->tree_groups)
+        std::stable_sort(list.begin(), list.end(), [&](int32_t x, int32_t y) {
+            return c->sys[(size_t)c->groups[(size_t)x].sys].ndof > c->sys[(size_t)c->groups[(size_t)y].sys].ndof;
+        });
+    for (int m = 0; m < 2; ++m)
+        if ((rc = upload(c->d_tree_groups[m], c->tree_groups[m], c->stream))) return bail(rc);
+    if ((rc = upload(c->d_tree_scale, tree_scales, c->stream))) return bail(rc);
     for (int cls = 0; cls < 4; ++cls)
         if ((rc = upload(c->d_class_groups[cls], c->class_groups[cls], c->stream))) return bail(rc);
     for (int m = 0; m < 2; ++m)
@@ -863,6 +990,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
     for (int cls = 0; cls < 4; ++cls) c->class_groups_all[cls] = c->class_groups[cls];
     for (int m = 0; m < 2; ++m)
         for (int i = 0; i < 5; ++i) c->tuned_groups_all[m][i] = c->tuned_groups[m][i];
+    for (int m = 0; m < 2; ++m) c->tree_groups_all[m] = c->tree_groups[m];
     c->pairs_even_all = c->pairs_even;
     c->pairs_odd_all = c->pairs_odd;
     if ((rc = upload(c->d_w_flavor, flav, c->stream))) return bail(rc);
@@ -1064,6 +1192,10 @@ static int retire_done_systems(rewl_ctx* c) {
             keep(c->tuned_groups[m][i]);
             if ((rc = overwrite(c->d_tuned_groups[m][i], c->tuned_groups[m][i], c->stream))) return rc;
         }
+    for (int m = 0; m < 2; ++m) {
+        keep(c->tree_groups[m]);
+        if ((rc = overwrite(c->d_tree_groups[m], c->tree_groups[m], c->stream))) return rc;
+    }
     auto keep_pairs = [&](std::vector<int32_t>& pl) {
         std::vector<int32_t> out;
         for (int32_t w : pl)
@@ -1096,6 +1228,10 @@ static int unretire_all(rewl_ctx* c) {
             c->tuned_groups[m][i] = c->tuned_groups_all[m][i];
             if ((rc = overwrite(c->d_tuned_groups[m][i], c->tuned_groups[m][i], c->stream))) return rc;
         }
+    for (int m = 0; m < 2; ++m) {
+        c->tree_groups[m] = c->tree_groups_all[m];
+        if ((rc = overwrite(c->d_tree_groups[m], c->tree_groups[m], c->stream))) return rc;
+    }
     c->pairs_even = c->pairs_even_all;
     c->pairs_odd = c->pairs_odd_all;
     if ((rc = overwrite(c->d_pairs_even, c->pairs_even, c->stream))) return rc;

@@ -312,7 +312,7 @@ namespace rewl {
 
 // Largest |T(k) - (-ln(k 2^-32))| over k = base + i, i < n (k = 0 skipped),
 // the error the acceptance band kLogBand has to cover.
-__global__ void k_selfcheck_neglog(uint32_t base, uint32_t n, unsigned long long* out_bits) {
+static __global__ void k_selfcheck_neglog(uint32_t base, uint32_t n, unsigned long long* out_bits) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     double err = 0.0;
     for (uint32_t j = i; j < n; j += gridDim.x * blockDim.x) {

@@ -1,0 +1,577 @@
+// Wang-Landau sweep, Philox mode, integer energies, a few thousand walkers at
+// most: sixteen lanes per walker.
+//
+// Same chain, same draws and the same FP64 ln g arithmetic as k_sweep (the
+// reference's wang_landau_update, wang_landau.hpp:49-93).  With one lane per
+// walker the chip is mostly idle and a walker's time per attempt is the length
+// of one wavefront's instruction stream plus an LDS read on its dependency
+// chain (158 cycles an attempt at L = 64).  Here a walker has a row of sixteen
+// lanes and takes four attempts at a time: the outcomes of four successive
+// attempts are a binary tree of fifteen decisions, each lane makes one of
+// them under the hypothesis that the attempts before it ended as its place in
+// the tree says, and the walk from the root along the decisions gives what
+// the four attempts in order give.  One LDS read latency and one state
+// hand-over are paid per four attempts instead of per attempt.
+//
+// A lane's node n (heap order: root 1, children 2n and 2n + 1) has depth t =
+// 0..3; bit a_i of n's path is the assumed outcome of attempt i < t.
+//
+//  * Row prologue: lane j of a walker's row takes block j (sites 4j..4j+3) of
+//    the lattice row, whose neighbours above, below and to the right are
+//    final (held in registers), and writes the energy changes of its four sites as signed bytes,
+//    for the left neighbour as it stands and flipped.  The lattice is kept in
+//    LDS as one nibble per byte, so a block is a byte.
+//  * A node picks its path's four bytes with one v_perm_b32 and gets its
+//    current and proposed state with one v_dot4_i32_i8 each: the state u is
+//    the LDS byte offset of ln g at the walker's energy (energy x pitch / bin,
+//    so the bin's slot is u with the low bits masked).
+//  * The increments of the path's earlier attempts are applied to the two
+//    ln g values in registers: one masked add of ln f for each earlier state
+//    in the same bin (the adds are all of the same ln f, so their order does
+//    not matter and the sums round as in sequence).
+//  * Guard bins hold ln g = +inf and reach four proposals beyond the window,
+//    so every hypothetical state is a valid slot, and one outside the window
+//    is rejected by the comparison itself.
+//  * The lanes on the walked path add ln f and a count to the bin after their
+//    attempt; the last one hands the state and the step's flips over to its
+//    row through an LDS word per block.
+//
+// The acceptance bounds come from producer wavefronts (accept_bound.hpp), a
+// segment of rows ahead, one barrier per segment.
+//
+// What bounds it: the instruction stream of one wavefront (about 5 cycles an
+// instruction when it has its SIMD to itself) and two LDS round trips per four
+// attempts.  Of the 440 cycles of a step the sixteen instructions of the
+// increments take 85, the FP64 atomic 50 and the count 25; a row adds 320.
+// Measured, cycles per attempt per walker, one lane a walker -> this kernel:
+// L = 64 Ising, 2048 walkers 158 -> 115 (270 -> 196 ms per 1000 sweeps); L = 16,
+// 8 walkers 253 -> 130; L = 42, 256 walkers (row kernel) 493 -> 112; L = 32
+// Ashkin-Teller, 512 walkers 196 -> 128.  Steps of three attempts cost 107 by
+// the same count and two 126; the spin flips as an LDS exclusive-or on the path
+// and the state hand-over before the updates measured no better.
+#pragma once
+#include "accept_bound.hpp"
+#include "device.hpp"
+#include "sweep_tuned.hpp"
+
+namespace rewl {
+
+constexpr int kTreeLanes = 16;      // lanes per walker
+constexpr int kTreePerWave = 4;     // walkers per wavefront
+constexpr int kTreeMaxDepth = 4;    // attempts per step
+constexpr int kTreeMinL = 5;        // the first and the last block of a row differ
+
+// Byte scale of one system's states and energy changes (host: tree_scale).
+struct TreeScale {
+    int32_t pitch;   // bytes of one ln g bin row in LDS (power of two, >= the bin size)
+    int32_t g;       // every energy change is a multiple of g
+    int32_t m;       // stored byte = energy change / g * m
+    int32_t w;       // state bytes per stored unit: w m = pitch g / bin
+    int32_t guard;   // guard bins on each side
+};
+
+// LDS of one workgroup of `nw` walker wavefronts (offsets in bytes).
+struct TreeLds {
+    int32_t rowb, lat, ring, ringw, rec, cnt, lng, total;
+};
+
+// Per walker: 16 records of a row's blocks and the last one's alternative
+// (8 bytes each), then 16 state words, one per block, and a sink of the same
+// size for the lanes that do not end a step.
+constexpr int kTreeAlt = 128, kTreeState = 136, kTreeSink = 264, kTreeRow = 392;
+
+constexpr __host__ __device__ int tree_blocks(int L) { return (L + 3) / 4; }
+// rows per segment of bounds: at least 32 attempts between barriers
+constexpr __host__ __device__ int tree_seg_rows(int L) { return L >= 32 ? 1 : (32 + L - 1) / L; }
+
+__host__ __device__ inline TreeLds tree_lds(int planes, int L, int nbins, int nw, int pitch, int guard) {
+    const int S = nw * kTreePerWave;
+    TreeLds t;
+    t.rowb = (tree_blocks(L) + 3) & ~3;                    // a row of nibbles
+    t.lat = 0;                                             // [walker][plane][row]
+    t.ringw = 2 * tree_seg_rows(L) * L * 8 + 32;           // bounds of one walker
+    t.ring = (t.lat + S * (planes * L * t.rowb + 4) + 15) & ~15;
+    t.rec = t.ring + S * t.ringw;                          // [walker] kTreeRow bytes, see there
+    const int other = t.rec + S * kTreeRow;
+    const int nb = nbins + 2 * guard;
+    // ln g at twice the offset of the counts, so that a count's address is
+    // half its ln g's
+    int cb = other > nb * pitch / 2 ? other : nb * pitch / 2;
+    cb = (cb + pitch - 1) & ~(pitch - 1);
+    t.cnt = cb;
+    t.lng = 2 * cb;
+    t.total = t.lng + nb * pitch;
+    return t;
+}
+
+typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) u32x2v lds_u32x2_t;
+typedef __attribute__((address_space(3))) uint8_t lds_u8_t;
+__device__ __forceinline__ u32x2v lds_u32x2(uint32_t addr) { return *(lds_u32x2_t*)(uintptr_t)addr; }
+__device__ __forceinline__ void lds_store_u32x2(uint32_t addr, u32x2v v) { *(lds_u32x2_t*)(uintptr_t)addr = v; }
+__device__ __forceinline__ uint32_t lds_u8(uint32_t addr) { return *(lds_u8_t*)(uintptr_t)addr; }
+__device__ __forceinline__ void lds_store_u8(uint32_t addr, uint32_t v) { *(lds_u8_t*)(uintptr_t)addr = (uint8_t)v; }
+
+// bit i of a nibble to bit 8 i
+__device__ __forceinline__ uint32_t spread_nibble(uint32_t x) { return __umul24(x, 0x204081u) & 0x01010101u; }
+
+// x + f if c, else x, rounded once (f finite)
+__device__ __forceinline__ double add_if(bool c, double f, double x) {
+    return __builtin_fma(__hiloint2double(c ? 0x3ff00000 : 0, 0), f, x);
+}
+
+// What a lane keeps for its node.
+struct TreeLane {
+    uint32_t sel0;              // v_perm selector of its path's bytes (left of the block's first site as it stands)
+    int wC, wN, w1, w2;         // byte weights: current state, proposal, states after the first and second attempt
+    double f1, f2, f3;          // ln f where that earlier state exists, else 0
+    uint32_t mlo, mhi;          // its ancestors' bits of the decision mask
+    uint32_t want, want_tail;   // their outcomes on its path (all ones: never on the path)
+    uint32_t out0, out1;        // outcomes word if its attempt is rejected, accepted: flips << 4, 4 if the last site flipped
+    uint32_t l8;                // its walker's column of ln g
+    double lnf;
+};
+
+struct TreeState {
+    uint32_t u;      // LDS offset of ln g at the walker's energy
+    uint32_t out;    // outcomes of the step before: bit 2 its last site flipped, bits 4..7 its sites' flips
+};
+
+// The states of a node and their slots: C, N = u + dv.w (signed bytes) and the
+// states after the path's first and second attempt, then each slot = (state &
+// mask) | l8.  One block, because the result of a dot product may be read by
+// another VALU instruction only three instructions later, which this order
+// keeps (and because the three-operand form leaves u where it is).
+__device__ __forceinline__ void node_slots(const TreeLane& c, uint32_t dv, uint32_t u, uint32_t mask, uint32_t& C,
+                                           uint32_t& N, uint32_t& sC, uint32_t& sN, uint32_t& s1, uint32_t& s2) {
+    asm("v_dot4_i32_i8 %[C], %[dv], %[wC], %[u]\n\t"
+        "v_dot4_i32_i8 %[N], %[dv], %[wN], %[u]\n\t"
+        "v_dot4_i32_i8 %[s1], %[dv], %[w1], %[u]\n\t"
+        "v_dot4_i32_i8 %[s2], %[dv], %[w2], %[u]\n\t"
+        "v_and_or_b32 %[sC], %[C], %[mask], %[l8]\n\t"
+        "v_and_or_b32 %[sN], %[N], %[mask], %[l8]\n\t"
+        "v_and_or_b32 %[s1], %[s1], %[mask], %[l8]\n\t"
+        "v_and_or_b32 %[s2], %[s2], %[mask], %[l8]"
+        : [C] "=&v"(C), [N] "=&v"(N), [sC] "=&v"(sC), [sN] "=&v"(sN), [s1] "=&v"(s1), [s2] "=&v"(s2)
+        : [dv] "v"(dv), [wC] "v"(c.wC), [wN] "v"(c.wN), [w1] "v"(c.w1), [w2] "v"(c.w2), [u] "v"(u), [mask] "s"(mask),
+          [l8] "v"(c.l8));
+}
+
+struct TreeInput {
+    u32x2v rec;   // energy-change bytes of the block's sites, left neighbour as it stands / flipped
+    double B;     // acceptance bound of this lane's attempt
+};
+
+// Four attempts (or, TAIL, the row's last r < 4: lanes of deeper nodes have
+// want_tail = never).  `in` is the block's input on entry; the next block's,
+// read from next_rec and next_B while this one's ln g are in flight, on exit.
+// The state goes to au + AT (the row's word for the lane that ends the step,
+// else the sink) and is read back from ust + AT by the whole row.
+template <bool TAIL, int AT>
+__device__ __forceinline__ void tree_block(const TreeLane& c, TreeState& st, TreeInput& in, uint32_t next_rec,
+                                           uint32_t next_B, uint32_t mask, uint32_t au, uint32_t ust) {
+    const uint32_t dv = __builtin_amdgcn_perm(in.rec.y, in.rec.x, c.sel0 | (st.out & 4u));
+    uint32_t C, N, sC, sN, s1, s2;
+    node_slots(c, dv, st.u, mask, C, N, sC, sN, s1, s2);
+    double lc = lds_f64(sC), ln = lds_f64(sN);
+    const double B = in.B;
+    if (!TAIL) {
+        in.rec = lds_u32x2(next_rec);
+        in.B = lds_f64(next_B);
+    }
+    lc = add_if(sC == s1, c.f1, lc);
+    ln = add_if(sN == s1, c.f1, ln);
+    lc = add_if(sC == s2, c.f2, lc);
+    ln = add_if(sN == s2, c.f2, ln);
+    lc = lc + c.f3;
+    ln = add_if(sN == sC, c.f3, ln);
+    const bool acc = (ln - lc) < B;
+    const uint64_t M = __builtin_amdgcn_ballot_w64(acc);
+    const uint32_t pv = ((uint32_t)M & c.mlo) | ((uint32_t)(M >> 32) & c.mhi);
+    const uint64_t path = __builtin_amdgcn_ballot_w64(pv == (TAIL ? c.want_tail : c.want));
+    u32x2v uf;
+    uf.x = acc ? N : C;
+    uf.y = acc ? c.out1 : c.out0;
+    const uint32_t sF = acc ? sN : sC;
+    const uint32_t cF = sF >> 1, one = 1u;
+    // The last lane of the path hands the state over to its row; the lanes on
+    // the path add ln f and a count.  (Stores and atomics without return;
+    // every lane is active here.)
+    asm volatile("s_mov_b64 exec, %[path]\n\t"
+                 "ds_write_b64 %[au], %[uf] offset:%[at]\n\t"
+                 "ds_add_f64 %[sF], %[lnf]\n\t"
+                 "ds_add_u32 %[cF], %[one]\n\t"
+                 "s_mov_b64 exec, -1"
+                 :
+                 : [path] "s"(path), [au] "v"(au), [uf] "v"(uf), [at] "n"(AT), [sF] "v"(sF), [lnf] "v"(c.lnf),
+                   [cF] "v"(cF), [one] "v"(one)
+                 : "memory");
+    const u32x2v s = lds_u32x2(ust + AT);
+    st.u = s.x;
+    st.out = s.y;
+}
+
+// One walker wavefront: walkers 4 wave .. 4 wave + 3 of the group.
+template <int MODEL>
+__device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGroup& G, const DevSystem& S,
+                                                   const TreeScale& T, const TreeLds& o, int wave, int nsweeps) {
+    using Mdl = Model<MODEL>;
+    constexpr int NP = Mdl::kPlanes;
+    constexpr int NPASS = Mdl::kPasses;
+    constexpr bool KQ = Mdl::kProductCoupling;
+    const int tid = threadIdx.x & 63;
+    const int n = tid & 15, row = tid >> 4;
+    const int j = kTreePerWave * wave + row;
+    const bool active = j < G.nwalkers;
+    const int g = G.first_walker + (active ? j : 0);
+    const DevWindow Wn = a.win[a.w_window[g]];
+    const double lnf = a.win_lnf[a.w_window[g]];
+    const int L = S.L, nblk = tree_blocks(L), tail = L - 4 * (nblk - 1);
+    const uint32_t mask = ~(uint32_t)(T.pitch - 1);
+    const int bshift = Wn.shift;                                  // log2 of the bin size
+    const int pshift = 31 - __builtin_clz((unsigned)T.pitch);
+    const uint32_t u0 = (uint32_t)(o.lng + T.guard * T.pitch);    // energy = window minimum
+
+    // ---- the lane's node -----------------------------------------------------
+    TreeLane c;
+    {
+        const int t = n < 2 ? 0 : n < 4 ? 1 : n < 8 ? 2 : 3;
+        uint32_t anc = 0, want = 0, sel = 0x03020100u;
+        int wC = 0, w1 = 0, w2 = 0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            if (i >= t) continue;
+            const int k = t - i;              // the ancestor that decides attempt i is n >> k
+            const int ai = (n >> (k - 1)) & 1;
+            anc |= 1u << (n >> k);
+            want |= (uint32_t)ai << (n >> k);
+            if (ai) {
+                wC |= T.w << (8 * i);
+                if (i < 1 && t >= 2) w1 |= T.w << (8 * i);
+                if (i < 2 && t >= 3) w2 |= T.w << (8 * i);
+                sel |= 4u << (8 * (i + 1));   // the site after a flip sees its left neighbour flipped
+            }
+        }
+        c.sel0 = sel;
+        c.wC = wC;
+        c.wN = wC | (T.w << (8 * t));
+        c.w1 = w1;
+        c.w2 = w2;
+        c.f1 = t >= 2 ? lnf : 0.0;
+        c.f2 = t >= 3 ? lnf : 0.0;
+        c.f3 = t >= 1 ? lnf : 0.0;
+        const uint32_t sh = 16u * (row & 1);
+        const bool on = active && n > 0;
+        c.mlo = on && row < 2 ? anc << sh : 0u;
+        c.mhi = on && row >= 2 ? anc << sh : 0u;
+        c.want = on ? want << sh : 0xffffffffu;
+        c.want_tail = on && t < tail ? want << sh : 0xffffffffu;
+        uint32_t flips = 0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            if (i < t) flips |= (uint32_t)((n >> (t - i - 1)) & 1) << (4 + i);
+        c.out0 = flips;
+        c.out1 = flips | (1u << (4 + t)) | 4u;
+        c.l8 = (uint32_t)(j * 8);
+        c.lnf = lnf;
+    }
+    const int depth = n < 2 ? 0 : n < 4 ? 1 : n < 8 ? 2 : 3;
+    const uint32_t latw = (uint32_t)(o.lat + j * (NP * L * o.rowb + 4));
+    const uint32_t recw = (uint32_t)(o.rec + j * kTreeRow);
+    // where the lane leaves a step's state: the row's word if it ends the step
+    const uint32_t au = recw + (uint32_t)(depth == 3 ? kTreeState : kTreeSink);
+    const uint32_t au_tail = recw + (uint32_t)(depth == tail - 1 ? kTreeState : kTreeSink);
+    const uint32_t ringw = (uint32_t)(o.ring + j * o.ringw + depth * 8);
+    // energy change bytes by the number of disagreeing neighbours; with two
+    // couplings biased by 64 each, so that the bytes add without carries, and
+    // made signed afterwards
+    uint32_t tj_lo = 0, tj_hi = 0, tk_lo = 0, tk_hi = 0;
+    {
+        auto entry = [&](int two, int k) { return (uint32_t)((two * (4 - 2 * k) / T.g) * T.m + (KQ ? 64 : 0)) & 255u; };
+        for (int k = 0; k < 4; ++k) {
+            tj_lo |= entry(S.twoJ, k) << (8 * k);
+            if (KQ) tk_lo |= entry(S.twoK, k) << (8 * k);
+        }
+        tj_hi = entry(S.twoJ, 4);
+        if (KQ) tk_hi = entry(S.twoK, 4);
+    }
+    int fl = a.w_flavor[g];
+    // the walker is inside its window (rewl_adjust_to_range); the clamp keeps
+    // its slot in bounds regardless
+    const int e0 = min(max((int)a.w_E[g] - Wn.imin, 0), (Wn.nbins << bshift) - 1);
+    TreeState st{u0 + (uint32_t)(e0 << (pshift - bshift)), 0u};
+    // an absent walker's row never writes its state words
+    if (n < nblk) lds_store_u32x2(recw + (uint32_t)(kTreeState + 8 * n), u32x2v{st.u, 0u});
+
+    // the lane's block of a row and its neighbours in the row
+    const int b = n < nblk ? n : nblk - 1;
+    const int bl = b == 0 ? nblk - 1 : b - 1, br = b == nblk - 1 ? 0 : b + 1;
+    const int topl = bl == nblk - 1 ? tail - 1 : 3, top = b == nblk - 1 ? tail - 1 : 3;
+    // Counts of disagreeing neighbours below and beside, by site of the lane's
+    // block: [right neighbour of the row's last site as it stands, flipped]
+    // [left neighbour as it stands, flipped]; the product plane's too.
+    struct Beside {
+        uint32_t p[2][2], q[2][2];
+    } bs{};
+    uint32_t up = 0, cur = 0, dn = 0;   // the lane's nibbles: the row above as rewritten, this row, the row below
+    uint32_t qcu = 0;                   // product coupling: other plane's disagreement with the row above
+    uint32_t lat = 0, latq = 0;         // the plane this pass flips, the other one
+    struct Bytes {
+        uint32_t dn, l, r, qc, qu, qd, ql, qr;
+    };
+    // row y's bytes around the lane's block (its own nibble aside)
+    auto read_row = [&](int y) {
+        const int yd = y == L - 1 ? 0 : y + 1;
+        Bytes v{};
+        v.dn = lds_u8(lat + (uint32_t)(yd * o.rowb + b));
+        v.l = lds_u8(lat + (uint32_t)(y * o.rowb + bl));
+        v.r = lds_u8(lat + (uint32_t)(y * o.rowb + br));
+        if constexpr (KQ) {
+            const int yu = y == 0 ? L - 1 : y - 1;
+            v.qc = lds_u8(latq + (uint32_t)(y * o.rowb + b));
+            v.qu = lds_u8(latq + (uint32_t)(yu * o.rowb + b));
+            v.qd = lds_u8(latq + (uint32_t)(yd * o.rowb + b));
+            v.ql = lds_u8(latq + (uint32_t)(y * o.rowb + bl));
+            v.qr = lds_u8(latq + (uint32_t)(y * o.rowb + br));
+        }
+        return v;
+    };
+    // disagreements of nibble p with the site to the right, to the left
+    auto right_of = [&](uint32_t p, uint32_t r) { return p ^ ((p >> 1) | ((r & 1u) << top)); };
+    auto left_of = [&](uint32_t p, uint32_t l) { return (p ^ ((p << 1) | ((l >> topl) & 1u))) & 15u; };
+    auto beside = [&](uint32_t p, const Bytes& v) {
+        const uint32_t rt = right_of(p, v.r), lf = left_of(p, v.l), d = p ^ v.dn;
+        auto sums = [&](uint32_t dd, uint32_t rr, uint32_t ll, uint32_t (&out)[2][2]) {
+            const uint32_t s = spread_nibble(dd), r0 = spread_nibble(rr), r1 = r0 ^ (1u << (8 * top));
+            const uint32_t l0 = spread_nibble(ll), l1 = l0 ^ 0x01010101u;
+            out[0][0] = s + r0 + l0;
+            out[0][1] = s + r0 + l1;
+            out[1][0] = s + r1 + l0;
+            out[1][1] = s + r1 + l1;
+        };
+        sums(d, rt, lf, bs.p);
+        if constexpr (KQ) {
+            sums(d ^ v.qc ^ v.qd, rt ^ right_of(v.qc, v.qr), lf ^ left_of(v.qc, v.ql), bs.q);
+            qcu = v.qc ^ v.qu;
+        }
+        dn = v.dn;
+    };
+    const bool last_block = n >= nblk - 1;
+    const int seg_rows = tree_seg_rows(L);
+    const int nrows = nsweeps * NPASS * L;
+    int y = 0, in_seg = 0, slot = 0;
+    __syncthreads();   // LDS loaded, first segment of bounds ready
+    for (int r = 0; r < nrows; ++r) {
+        if (y == 0 && (NPASS > 1 || r == 0)) {
+            const int pf = Mdl::flip_plane(fl), qf = NP - 1 - pf;
+            lat = latw + (uint32_t)(pf * L * o.rowb);
+            latq = latw + (uint32_t)(qf * L * o.rowb);
+            up = lds_u8(lat + (uint32_t)((L - 1) * o.rowb + b));
+            cur = lds_u8(lat + b);
+            beside(cur, read_row(0));
+        }
+        const uint32_t ring = ringw + (uint32_t)(slot * L * 8);
+        TreeInput in;
+        in.B = lds_f64(ring);
+        // ---- energy changes of the row: lane n takes block n; only the row
+        // above is new, the rest was prepared during the row before ------------
+        const uint32_t su = spread_nibble(cur ^ up);
+        uint32_t sq = 0;
+        if constexpr (KQ) sq = spread_nibble(cur ^ up ^ qcu);
+        auto record = [&](int alt) {
+            u32x2v v;
+            v.x = __builtin_amdgcn_perm(tj_hi, tj_lo, su + bs.p[alt][0]);
+            v.y = __builtin_amdgcn_perm(tj_hi, tj_lo, su + bs.p[alt][1]);
+            if constexpr (KQ) {
+                v.x += __builtin_amdgcn_perm(tk_hi, tk_lo, sq + bs.q[alt][0]);
+                v.y += __builtin_amdgcn_perm(tk_hi, tk_lo, sq + bs.q[alt][1]);
+                v ^= 0x80808080u;
+            }
+            return v;
+        };
+        {
+            const u32x2v v = record(0);
+            if (n < nblk) lds_store_u32x2(recw + 8u * (uint32_t)n, v);
+            // the first block's: lane 0's, to its row
+            in.rec.x = (uint32_t)__builtin_amdgcn_mov_dpp((int)v.x, 0x150, 0xf, 0xf, false);
+            in.rec.y = (uint32_t)__builtin_amdgcn_mov_dpp((int)v.y, 0x150, 0xf, 0xf, false);
+        }
+        const Bytes nx = read_row(y == L - 1 ? 0 : y + 1);
+        // ---- the row's blocks --------------------------------------------------
+        st.out = 0u;   // left of site 0 is site L - 1, as it stands
+        const uint32_t nlast = (uint32_t)(nblk - 1);
+        // blocks q4 + k, k = 0..3, in fours from q4 = 0
+        uint32_t x = recw, rg = ring, aq = au;   // addresses at block q4
+        asm("" : "+v"(x), "+v"(rg), "+v"(aq));
+        tree_block<false, 0>(c, st, in, x + 8u, rg + 32u, mask, aq, x + (uint32_t)kTreeState);
+        if (n == nblk - 1) lds_store_u32x2(recw + (uint32_t)kTreeAlt, record(1));
+        const uint32_t own = cur;
+        cur = dn;
+        beside(cur, nx);   // for the next row
+        // the last block's last site sees site 0 as it is now
+        const uint32_t rec_last = (st.out & 16u) ? recw + (uint32_t)kTreeAlt : recw + 8u * nlast;
+        auto next_rec = [&](uint32_t i, uint32_t xr) { return i == nlast ? rec_last : xr; };
+        if (nlast > 1u) tree_block<false, 8>(c, st, in, next_rec(2u, x + 16u), rg + 64u, mask, aq, x + (uint32_t)kTreeState);
+        if (nlast > 2u) tree_block<false, 16>(c, st, in, next_rec(3u, x + 24u), rg + 96u, mask, aq, x + (uint32_t)kTreeState);
+        if (nlast > 3u) tree_block<false, 24>(c, st, in, next_rec(4u, x + 32u), rg + 128u, mask, aq, x + (uint32_t)kTreeState);
+        uint32_t i = 4u;
+        x += 32u;
+        rg += 128u;
+        aq += 32u;
+        for (; i + 4u <= nlast; i += 4u) {
+            // opaque, so that every address of the four is one of these plus
+            // an offset of its instruction
+            asm("" : "+v"(x), "+v"(rg), "+v"(aq));
+            tree_block<false, 0>(c, st, in, x + 8u, rg + 32u, mask, aq, x + (uint32_t)kTreeState);
+            tree_block<false, 8>(c, st, in, x + 16u, rg + 64u, mask, aq, x + (uint32_t)kTreeState);
+            tree_block<false, 16>(c, st, in, x + 24u, rg + 96u, mask, aq, x + (uint32_t)kTreeState);
+            tree_block<false, 24>(c, st, in, next_rec(i + 4u, x + 32u), rg + 128u, mask, aq, x + (uint32_t)kTreeState);
+            x += 32u;
+            rg += 128u;
+            aq += 32u;
+        }
+        if (i < nlast) {
+            asm("" : "+v"(x), "+v"(rg), "+v"(aq));
+            tree_block<false, 0>(c, st, in, next_rec(i + 1u, x + 8u), rg + 32u, mask, aq, x + (uint32_t)kTreeState);
+            if (i + 1u < nlast)
+                tree_block<false, 8>(c, st, in, next_rec(i + 2u, x + 16u), rg + 64u, mask, aq, x + (uint32_t)kTreeState);
+            if (i + 2u < nlast)
+                tree_block<false, 16>(c, st, in, next_rec(i + 3u, x + 24u), rg + 96u, mask, aq, x + (uint32_t)kTreeState);
+        }
+        if (nlast == 1u) in.rec = lds_u32x2(rec_last);   // read before the first block was decided
+        // ---- the row as rewritten: the state words hold the blocks' flips ----
+        const uint32_t word = lds_u32x2(recw + (uint32_t)(kTreeState + 8 * b)).y;
+        tree_block<true, 0>(c, st, in, 0u, 0u, mask, au_tail + 8u * nlast, recw + 8u * nlast + (uint32_t)kTreeState);
+        up = own ^ (((last_block ? st.out : word) >> 4) & 15u);
+        if (n < nblk) lds_store_u8(lat + (uint32_t)(y * o.rowb + n), up);
+        if (++y == L) {
+            y = 0;
+            fl = Mdl::next_flavour(fl);   // flavour switches after site N - 1
+        }
+        if (++slot == 2 * seg_rows) slot = 0;
+        if (++in_seg == seg_rows) {
+            in_seg = 0;
+            __syncthreads();   // this segment's bounds consumed, the next one's written
+        }
+    }
+    if (in_seg) __syncthreads();
+    if (active && n == 0) {
+        a.w_E[g] = (double)((int)((st.u - u0) >> (pshift - bshift)) + Wn.imin);
+        a.w_flavor[g] = fl;
+    }
+}
+
+// Producer side: the bounds of the rows [r0, r0 + count) (rows of the launch,
+// counted over its passes and sweeps) for every walker of the group, one
+// Philox block (up to four bounds) per lane.
+template <int MODEL>
+__device__ __forceinline__ void tree_fill(const DevGroup& G, const DevSystem& S, const TreeLds& o, int ptid, int nthreads,
+                                          uint64_t sweep_base, int r0, int count, int nwpad, const BoundEntry* tab) {
+    const int L = S.L, per_sweep = Model<MODEL>::kPasses * L;
+    const uint64_t blocks = (uint64_t)((S.ndof + 3) / 4);   // Philox blocks per sweep
+    const int nbb = (L & 3) ? L / 4 + 2 : L / 4;            // blocks that a row can touch
+    const int seg2 = 2 * tree_seg_rows(L);
+    const int total = count * nbb * nwpad;
+    for (int i = ptid; i < total; i += nthreads) {
+        const int j = i & (nwpad - 1);
+        const int rest = i / nwpad;
+        const int k = rest / nbb, bb = rest - k * nbb;
+        if (j >= G.nwalkers) continue;
+        const int r = r0 + k;
+        const int s = r / per_sweep;
+        const int p0 = (r - s * per_sweep) * L;             // attempt position of the row's first site in its sweep
+        const int blk = (p0 >> 2) + bb;
+        const int x0 = 4 * blk - p0;
+        if (x0 >= L) continue;
+        const uint64_t bi = (sweep_base + (uint64_t)s) * blocks + (uint64_t)blk;
+        const uint32_t walker = (uint32_t)(G.first_walker - S.first_walker + j);
+        const u32x4 w = philox4x32_10(u32x4{(uint32_t)bi, (uint32_t)(bi >> 32), DOMAIN_SWEEP, walker}, S.k0, S.k1);
+        const double v[4] = {accept_bound(w.x, tab), accept_bound(w.y, tab), accept_bound(w.z, tab),
+                             accept_bound(w.w, tab)};
+        const uint32_t dst = (uint32_t)(o.ring + j * o.ringw + (r % seg2) * L * 8);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int x = x0 + q;
+            if (x >= 0 && x < L) lds_store_f64(dst + 8u * (uint32_t)x, v[q]);
+        }
+    }
+}
+
+// One workgroup = nw walker wavefronts (four walkers each) + producer
+// wavefronts; groups are taken persistently in blockIdx order.
+template <int MODEL>
+__global__ void __launch_bounds__(512) k_sweep_tree(KArgs a, const TreeScale* scale, const int32_t* groups, int ngroups,
+                                                    int nsweeps, uint64_t sweep_base, int nw) {
+    using Mdl = Model<MODEL>;
+    constexpr int NP = Mdl::kPlanes;
+    const int tid = threadIdx.x, nth = blockDim.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int SW = nw * kTreePerWave;
+    const BoundEntry* tab = static_cast<const BoundEntry*>(a.bound_tab);
+    if (wave < nw) __builtin_amdgcn_s_setprio(3);
+    for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x) {
+        const DevGroup G = a.grp[groups[gi]];
+        const DevSystem S = a.sys[G.sys];
+        const TreeScale T = scale[G.sys];
+        const int L = S.L;
+        const TreeLds o = tree_lds(NP, L, G.nbins, nw, T.pitch, T.guard);
+        // ---- load (LDS addresses are offsets: the kernel has no static LDS):
+        // histograms (guard bins and absent walkers: +inf), lattice --
+        const int nb = G.nbins + 2 * T.guard;
+        for (int i = tid; i < nb * SW; i += nth) {
+            const int j = i & (SW - 1), b = i / SW - T.guard;
+            const bool in = j < G.nwalkers && b >= 0 && b < a.win[a.w_window[G.first_walker + (j < G.nwalkers ? j : 0)]].nbins;
+            const int64_t h = G.hist_base + j + (int64_t)b * kLanes;
+            const uint32_t at = (uint32_t)((b + T.guard) * T.pitch + j * 8);
+            lds_store_f64((uint32_t)o.lng + at, in ? a.lng[h] : __builtin_inf());
+            lds_store_u32((uint32_t)o.cnt + at / 2, in ? a.cnt[h] : 0u);
+        }
+        for (int i = tid; i < NP * L * SW; i += nth) {
+            const int j = i & (SW - 1), qy = i / SW;
+            const uint64_t w = j < G.nwalkers ? a.lat[G.lat_base + j + (int64_t)qy * kLanes] : 0ull;
+            const uint32_t dst = (uint32_t)(o.lat + j * (NP * L * o.rowb + 4) + qy * o.rowb);
+            for (int k = 0; k < o.rowb / 4; ++k) {
+                const uint32_t x = (uint32_t)(w >> (16 * k)) & 0xffffu;
+                lds_store_u32(dst + 4u * (uint32_t)k,
+                              (x & 0xfu) | ((x & 0xf0u) << 4) | ((x & 0xf00u) << 8) | ((x & 0xf000u) << 12));
+            }
+        }
+        if (wave < nw) {
+            sweep_walkers_tree<MODEL>(a, G, S, T, o, wave, nsweeps);
+        } else {
+            const int nrows = nsweeps * Mdl::kPasses * L, seg = tree_seg_rows(L);
+            const int pt = tid - 64 * nw, pn = nth - 64 * nw;
+            tree_fill<MODEL>(G, S, o, pt, pn, sweep_base, 0, min(seg, nrows), SW, tab);
+            __syncthreads();   // pairs with the walkers' barrier after the load
+            for (int r = 0; r < nrows; r += seg) {
+                const int next = r + seg;
+                if (next < nrows) tree_fill<MODEL>(G, S, o, pt, pn, sweep_base, next, min(seg, nrows - next), SW, tab);
+                __syncthreads();   // pairs with the walkers' end-of-segment barrier
+            }
+        }
+        __syncthreads();   // the walkers' last updates are in LDS
+        // ---- store -----------------------------------------------------------
+        for (int i = tid; i < G.nbins * SW; i += nth) {
+            const int j = i & (SW - 1), b = i / SW;
+            if (j >= G.nwalkers || b >= a.win[a.w_window[G.first_walker + j]].nbins) continue;
+            const int64_t h = G.hist_base + j + (int64_t)b * kLanes;
+            const uint32_t at = (uint32_t)((b + T.guard) * T.pitch + j * 8);
+            a.lng[h] = lds_f64((uint32_t)o.lng + at);
+            a.cnt[h] = lds_u32_at((uint32_t)o.cnt + at / 2);
+        }
+        for (int i = tid; i < NP * L * SW; i += nth) {
+            const int j = i & (SW - 1), qy = i / SW;
+            if (j >= G.nwalkers) continue;
+            const uint32_t src = (uint32_t)(o.lat + j * (NP * L * o.rowb + 4) + qy * o.rowb);
+            uint64_t w = 0;
+            for (int k = 0; k < o.rowb / 4; ++k) {
+                const uint32_t v = lds_u32_at(src + 4u * (uint32_t)k);
+                w |= (uint64_t)((v & 0xfu) | ((v >> 4) & 0xf0u) | ((v >> 8) & 0xf00u) | ((v >> 12) & 0xf000u)) << (16 * k);
+            }
+            a.lat[G.lat_base + j + (int64_t)qy * kLanes] = w;
+        }
+        __syncthreads();   // LDS is reused by the next group
+    }
+}
+
+}  // namespace rewl

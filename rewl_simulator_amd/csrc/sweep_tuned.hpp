@@ -627,7 +627,7 @@ __global__ void __launch_bounds__(512) k_sweep_tuned(KArgs a, const int32_t* gro
 }
 
 // B(k) for k = ks[i] (the sweep kernel's acceptance bounds, device log)
-__global__ void k_selfcheck_bounds(const uint32_t* ks, uint32_t n, const BoundEntry* tab, double* out) {
+static __global__ void k_selfcheck_bounds(const uint32_t* ks, uint32_t n, const BoundEntry* tab, double* out) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
         out[i] = accept_bound(ks[i], tab);
 }
