@@ -1654,6 +1654,22 @@ int rewl_stitch(rewl_ctx* c, int32_t si, double states_per_site, double* energie
     return REWL_OK;
 }
 
+// Every energy below 1e100 and every temperature between 1e-100 and 1e100 in
+// size: E/T can be taken as a corrected product (ThermoT).
+static bool thermo_tame(const double* E, int32_t nb, double tmin, double tmax) {
+    const double lo = std::min(tmin, tmax), hi = std::max(tmin, tmax);
+    if (!(lo > 1e-100 && hi < 1e100) && !(hi < -1e-100 && lo > -1e100)) return false;
+    for (int32_t b = 0; b < nb; ++b)
+        if (!(std::fabs(E[b]) < 1e100)) return false;
+    return true;
+}
+
+static void launch_thermo(bool tame, const double* dE, const double* dl, int nb, int N, double tmin, double dT, int nT,
+                          double* dout) {
+    hipLaunchKernelGGL(tame ? k_thermo<true> : k_thermo<false>, dim3((unsigned)((nT + kThermoT - 1) / kThermoT)),
+                       dim3(kThermoT * kThermoWaves), 0, nullptr, dE, dl, nb, N, tmin, dT, nT, dout);
+}
+
 int rewl_thermodynamics(const double* E, const double* lng, int32_t nb, int32_t N, double tmin, double tmax, int32_t nT,
                         double* out) {
     if (!E || !lng || !out || nb < 2 || nT < 1 || N < 1) return fail(REWL_ERR_INVALID, "bad arguments");
@@ -1666,7 +1682,7 @@ int rewl_thermodynamics(const double* E, const double* lng, int32_t nb, int32_t 
     HIP_TRY(hipMemcpy(dE, E, (size_t)nb * sizeof(double), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dl, lng, (size_t)nb * sizeof(double), hipMemcpyHostToDevice));
     const double dT = (tmax - tmin) / (double)nT;
-    hipLaunchKernelGGL(k_thermo, dim3((nT + 127) / 128), dim3(128), 0, nullptr, dE, dl, nb, N, tmin, dT, nT, dout);
+    launch_thermo(thermo_tame(E, nb, tmin, tmax), dE, dl, nb, N, tmin, dT, nT, dout);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpy(out, dout, (size_t)nT * 5 * sizeof(double), hipMemcpyDeviceToHost));
     (void)hipFree(dE);
@@ -1727,7 +1743,7 @@ int rewl_thermodynamics_noalloc(const double* E, const double* lng, int32_t nb, 
     HIP_TRY(hipMemcpy(dE, E, (size_t)nb * sizeof(double), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dl, lng, (size_t)nb * sizeof(double), hipMemcpyHostToDevice));
     const double dT = (tmax - tmin) / (double)nT;
-    hipLaunchKernelGGL(k_thermo, dim3((nT + 127) / 128), dim3(128), 0, nullptr, dE, dl, nb, N, tmin, dT, nT, dout);
+    launch_thermo(thermo_tame(E, nb, tmin, tmax), dE, dl, nb, N, tmin, dT, nT, dout);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpy(out, dout, (size_t)nT * 5 * sizeof(double), hipMemcpyDeviceToHost));
     return REWL_OK;
@@ -1753,8 +1769,10 @@ int rewl_thermo_observables(const double* E, const double* lng, const double* ob
     if (e == hipSuccess) e = hipMemcpy(dobs, obs, (size_t)nb * nobs * sizeof(double), hipMemcpyHostToDevice);
     if (e == hipSuccess) {
         const double dT = (tmax - tmin) / (double)nT;
-        hipLaunchKernelGGL(k_thermo_obs, dim3((nT + 127) / 128), dim3(128), 0, nullptr, dE, dl, dobs, nb, nobs, tmin,
-                           dT, nT, dout);
+        hipLaunchKernelGGL(thermo_tame(E, nb, tmin, tmax) ? k_thermo_obs<true> : k_thermo_obs<false>,
+                           dim3((unsigned)((nT + kThermoT - 1) / kThermoT)), dim3(kThermoT * kThermoWaves), 0, nullptr,
+                           (const double*)dE, (const double*)dl, (const double*)dobs, (int)nb, (int)nobs, tmin, dT, (int)nT,
+                           dout);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpy(out, dout, (size_t)nT * nobs * sizeof(double), hipMemcpyDeviceToHost);
