@@ -2336,7 +2336,7 @@ int rewl_mlp_gradient(rewl_mlp* m, const float* x, const float* t, const float* 
     HIP_TRY(hipEventRecord(m->ev0, m->stream));
     hipLaunchKernelGGL(k_mlp<true>, dim3(G), dim3(256), 0, m->stream, a);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((NPART + 255) / 256), dim3(256), 0, m->stream, m->part, G, m->grad);
+    hipLaunchKernelGGL(k_mlp_reduce, dim3((NPART + 63) / 64), dim3(64), 0, m->stream, m->part, G, m->grad);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(m->ev1, m->stream));
     std::vector<float> g(NPART);
@@ -2380,17 +2380,14 @@ int rewl_mlp_train(rewl_mlp* m, const float* x, const float* t, const float* w, 
     for (int64_t s = 0; s < p->steps; ++s) {
         a.step = (uint64_t)s;
         hipLaunchKernelGGL(k_mlp<true>, dim3(G), dim3(256), 0, m->stream, a);
-        hipLaunchKernelGGL(k_mlp_reduce, dim3((NPART + 255) / 256), dim3(256), 0, m->stream, m->part, G, m->grad);
-        if (dloss)
-            HIP_TRY(hipMemcpyAsync(dloss + s, m->grad + NP, sizeof(float), hipMemcpyDeviceToDevice, m->stream));
         m->adam_t += 1;
         double lr = p->lr_final + 0.5 * (p->lr - p->lr_final) * (1.0 + std::cos(M_PI * (double)s / (double)std::max<int64_t>(1, p->steps)));
         if (s < p->warmup) lr *= (double)(s + 1) / (double)p->warmup;
         const double bc1 = 1.0 - std::pow(p->beta1, (double)m->adam_t);
         const double bc2 = 1.0 - std::pow(p->beta2, (double)m->adam_t);
-        hipLaunchKernelGGL(k_mlp_adam, dim3((NP + 255) / 256), dim3(256), 0, m->stream, m->theta, m->adam_m,
-                           m->adam_v, m->grad, (float)lr, (float)p->beta1, (float)p->beta2, (float)p->eps, (float)bc1,
-                           (float)bc2, m->wq);
+        hipLaunchKernelGGL(k_mlp_step, dim3((NPART + 63) / 64), dim3(64), 0, m->stream, (const float*)m->part, G, m->theta,
+                           m->adam_m, m->adam_v, (float)lr, (float)p->beta1, (float)p->beta2, (float)p->eps, (float)bc1,
+                           (float)bc2, m->wq, dloss ? dloss + s : nullptr);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) {
             if (dloss) (void)hipFree(dloss);

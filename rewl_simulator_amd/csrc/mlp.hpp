@@ -19,6 +19,12 @@
 // dW2 and dW3 accumulate in MFMA accumulators across a workgroup's tiles (K =
 // points); every workgroup writes one partial gradient and a second kernel
 // sums the partials in a fixed order (deterministic) and applies Adam.
+//
+// A training step of 8192 points is 256 tiles, one per CU: 31 us of one
+// wavefront per SIMD (48 error functions and exponentials a lane, then 34 MB of
+// partial gradients) and 11 us for the sum and Adam; 40, 63, 5 and a copy of
+// the loss before the error functions were kept for the backward pass, the
+// columns summed on the VALU and the steps after k_mlp made one.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -55,9 +61,13 @@ __host__ __device__ __forceinline__ float bf16_float(uint16_t b) {
     return __builtin_bit_cast(float, (uint32_t)b << 16);
 }
 
-__device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.707106781186547524f)); }
-__device__ __forceinline__ float gelu_grad(float z) {
-    const float cdf = 0.5f * (1.0f + erff(z * 0.707106781186547524f));
+// GELU and its derivative from e = 1 + erf(z / sqrt 2), which a training step
+// computes once per unit and point, in the forward pass, and keeps for the
+// backward pass.
+__device__ __forceinline__ float gelu_erf(float z) { return 1.0f + erff(z * 0.707106781186547524f); }
+__device__ __forceinline__ float gelu(float z, float e) { return 0.5f * z * e; }
+__device__ __forceinline__ float gelu_grad(float z, float e) {
+    const float cdf = 0.5f * e;
     const float pdf = expf(-0.5f * z * z) * 0.398942280401432678f;
     return cdf + z * pdf;
 }
@@ -68,6 +78,26 @@ __device__ __forceinline__ bf16x8 load8(const uint16_t* p) {
 
 __device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_of(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+// The sum over the 32 lanes of each half wavefront, pairs 16 apart first, then
+// 8, 4, 2, 1 apart, on the VALU: the other row of sixteen by a row swap, 8 and
+// 4 apart as rotations of the row (after the step before, a rotation and an
+// exchange reach equal values), 2 and 1 apart within quads.  As five shuffles
+// through LDS the sixteen sums of a tile took 2 us of its wavefront's time.
+__device__ __forceinline__ float sum_columns(float p) {
+    const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, p), __builtin_bit_cast(uint32_t, p),
+                                                     false, false);
+    p = __builtin_bit_cast(float, (uint32_t)sw[0]) + __builtin_bit_cast(float, (uint32_t)sw[1]);
+    p += dpp_of<0x128>(p);   // row_ror:8
+    p += dpp_of<0x124>(p);   // row_ror:4
+    p += dpp_of<0x4e>(p);    // quad_perm [2, 3, 0, 1]
+    p += dpp_of<0xb1>(p);    // quad_perm [1, 0, 3, 2]
+    return p;
 }
 
 struct Args {
@@ -150,13 +180,15 @@ __global__ void __launch_bounds__(256) k_mlp(Args a) {
         __syncthreads();
 
         // ---- layer 1 (VALU, D layout) ------------------------------------------
+        float e1[16], e2[16], e3[16];
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int b = drow(v, hf);
             float z = b1j;
 #pragma unroll
             for (int c = 0; c < NIN; ++c) z = z + w1j[c] * xs[b][c];
-            const uint16_t q = bf16_bits(gelu(z));
+            e1[v] = gelu_erf(z);
+            const uint16_t q = bf16_bits(gelu(z, e1[v]));
             a1r[b * RS + j] = q;
             a1t[j * TS + b] = q;
         }
@@ -176,7 +208,8 @@ __global__ void __launch_bounds__(256) k_mlp(Args a) {
         for (int v = 0; v < 16; ++v) {
             const int b = drow(v, hf);
             z2[v] = acc[v] + b2j;
-            const uint16_t q = bf16_bits(gelu(z2[v]));
+            e2[v] = gelu_erf(z2[v]);
+            const uint16_t q = bf16_bits(gelu(z2[v], e2[v]));
             a2r[b * RS + j] = q;
             a2t[j * TS + b] = q;
         }
@@ -193,9 +226,8 @@ __global__ void __launch_bounds__(256) k_mlp(Args a) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             z3[v] = acc[v] + b3j;
-            float p = w4j * gelu(z3[v]);
-#pragma unroll
-            for (int o = 16; o > 0; o >>= 1) p += __shfl_xor(p, o);   // over the 32 columns of this half
+            e3[v] = gelu_erf(z3[v]);
+            const float p = sum_columns(w4j * gelu(z3[v], e3[v]));   // over the 32 columns of this half
             if (lc == 0) yred[wv][drow(v, hf)] = p;
         }
         __syncthreads();
@@ -217,8 +249,8 @@ __global__ void __launch_bounds__(256) k_mlp(Args a) {
         for (int v = 0; v < 16; ++v) {
             const int b = drow(v, hf);
             const float dy = dys[b];
-            gw4 += dy * gelu(z3[v]);
-            const float dz = dy * w4j * gelu_grad(z3[v]);
+            gw4 += dy * gelu(z3[v], e3[v]);
+            const float dz = dy * w4j * gelu_grad(z3[v], e3[v]);
             gb3 += dz;
             const uint16_t q = bf16_bits(dz);
             dzr[b * RS + j] = q;
@@ -247,7 +279,7 @@ __global__ void __launch_bounds__(256) k_mlp(Args a) {
         float dz2[16];
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            dz2[v] = acc[v] * gelu_grad(z2[v]);
+            dz2[v] = acc[v] * gelu_grad(z2[v], e2[v]);
             gb2 += dz2[v];
         }
         __syncthreads();   // dz3 fully consumed
@@ -279,7 +311,7 @@ __global__ void __launch_bounds__(256) k_mlp(Args a) {
             float z1 = b1j;   // recomputed: the same operations as the forward pass
 #pragma unroll
             for (int c = 0; c < NIN; ++c) z1 = z1 + w1j[c] * xs[b][c];
-            const float dz1 = acc[v] * gelu_grad(z1);
+            const float dz1 = acc[v] * gelu_grad(z1, e1[v]);
             gb1 += dz1;
 #pragma unroll
             for (int c = 0; c < NIN; ++c) gw1[c] += dz1 * xs[b][c];
@@ -323,13 +355,28 @@ __global__ void __launch_bounds__(256) k_mlp(Args a) {
     }
 }
 
-// grad[p] = sum over partials g = 0..G-1 (in that order); p = NP is the loss.
+// The sum of parameter p's partials g = 0..G-1, in that order (p = NP is the
+// loss).  The loads of a run of partials go out together; one after the other
+// they cost 63 us a step at 256 partials, this way 11 us with Adam.
+constexpr int kReduceRun = 32;
+__device__ __forceinline__ float sum_partials(const float* part, int G, int p) {
+    float s = 0.f;
+    int g = 0;
+    for (; g + kReduceRun <= G; g += kReduceRun) {
+        float v[kReduceRun];
+#pragma unroll
+        for (int i = 0; i < kReduceRun; ++i) v[i] = part[(size_t)(g + i) * NPART + p];
+#pragma unroll
+        for (int i = 0; i < kReduceRun; ++i) s += v[i];
+    }
+    for (; g < G; ++g) s += part[(size_t)g * NPART + p];
+    return s;
+}
+
 __global__ void k_mlp_reduce(const float* part, int G, float* grad) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= NPART) return;
-    float s = 0.f;
-    for (int g = 0; g < G; ++g) s += part[(size_t)g * NPART + p];
-    grad[p] = s;
+    grad[p] = sum_partials(part, G, p);
 }
 
 __device__ __forceinline__ void store_quantised(uint16_t* wq, int p, float th) {
@@ -354,12 +401,19 @@ __global__ void k_mlp_quantise(const float* theta, uint16_t* wq) {
     if (p < NP) store_quantised(wq, p, theta[p]);
 }
 
-// Adam (Kingma & Ba) with bias correction; refreshes the bf16 copies.
-__global__ void k_mlp_adam(float* theta, float* m, float* v, const float* grad, float lr, float beta1, float beta2,
-                           float eps, float bc1, float bc2, uint16_t* wq) {
+// A training step after k_mlp: the gradient from the partials, Adam (Kingma &
+// Ba) with bias correction on it, the bf16 copies refreshed, and the step's
+// loss stored.
+__global__ void __launch_bounds__(64) k_mlp_step(const float* part, int G, float* theta, float* m, float* v, float lr,
+                                                 float beta1, float beta2, float eps, float bc1, float bc2, uint16_t* wq,
+                                                 float* loss) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= NP) return;
-    const float g = grad[p];
+    if (p >= NPART) return;
+    const float g = sum_partials(part, G, p);
+    if (p == NP) {
+        if (loss) *loss = g;
+        return;
+    }
     const float mp = beta1 * m[p] + (1.f - beta1) * g;
     const float vp = beta2 * v[p] + (1.f - beta2) * g * g;
     m[p] = mp;
