@@ -171,8 +171,11 @@ typedef struct rewl_params {
                                     kernel; 2 = row-unrolled; 3 = row-unrolled with
                                     the next slot computed for both outcomes; 4 =
                                     that and the next ln g read ahead (2-4 are an
-                                    error for other L or producers < 0).  Every
-                                    kernel runs the same chain                      */
+                                    error for other L or producers < 0).  FP64
+                                    energies (field models): 0 with producers = 0
+                                    and walkers_per_group = 0 = sixteen lanes per
+                                    walker in contexts of few walkers, else one.
+                                    Every kernel runs the same chain                */
     int32_t observables;         /* 1: per-bin observable sums of every update (each
                                     attempt and each post-exchange increment) at the
                                     walker's current bin: |m|, m^2, m^4 (Ising,

@@ -26,6 +26,7 @@
 #include "sweep_field.hpp"
 #include "sweep_tuned.hpp"
 #include "sweep_tree.hpp"
+#include "sweep_field_tree.hpp"
 #include "anneal.hpp"
 
 namespace rewl {
@@ -123,6 +124,17 @@ bool integral(double v) { return std::isfinite(v) && std::floor(v) == v && std::
 // Sizes without an unrolled-row kernel have the row kernel to compare with
 // (480-540 cycles): 215 at 8192, 389 at 12288.
 constexpr int kTreeMaxWalkers = 4096, kTreeMaxWalkersRow = 12288;
+// k_sweep_field_tree takes the FP64 systems of a context as long as their
+// walkers, each counted as its system's degrees of freedom over the largest
+// system's, are at most this many: 1024 workgroups, four per CU (registers and
+// LDS allow no more).  A second round of them takes as long as the kernel with
+// one lane per walker.  Measured, cycles per attempt, tree against lane: L = 30
+// random-field Ising 198 / 570 at 1024 walkers, 212 / 571 at 2048, 260 / 573 at
+// 4096, 643 / 570 at 8192; L = 32 186 / 441, 197 / 443, 243 / 442, 629 / 445;
+// L = 48 random-strain Ashkin-Teller 173 / 687, 222 / 687, 271 / 690, 615 / 693.
+// 8192 walkers of four sizes (16 to 48, 3698 counted so): 25.8 ms per 50 sweeps
+// against 73.9.
+constexpr int kFieldTreeMaxWalkers = 4096;
 
 constexpr int kTunedL[5] = {16, 24, 32, 48, 64};
 int tuned_index(int L) {
@@ -175,11 +187,12 @@ struct rewl_ctx {
     int tuned_guard[2][5] = {};                          // guard bins each side: max |Delta E| / bin size
     int tuned_nprod = 2;
     DevBuf<int32_t> d_tuned_groups[2][5];
-    // sixteen-lanes-a-walker kernel (sweep_tree.hpp): group lists per model
-    std::vector<int32_t> tree_groups[2], tree_groups_all[2];
-    DevBuf<int32_t> d_tree_groups[2];
+    // sixteen-lanes-a-walker kernels (sweep_tree.hpp, sweep_field_tree.hpp):
+    // group lists per model and energies (2 model + 1: FP64)
+    std::vector<int32_t> tree_groups[4], tree_groups_all[4];
+    DevBuf<int32_t> d_tree_groups[4];
     DevBuf<TreeScale> d_tree_scale;                      // per system
-    size_t tree_lds_bytes[2] = {0, 0};                   // the largest group's LDS
+    size_t tree_lds_bytes[4] = {0, 0, 0, 0};             // the largest group's LDS
     int tree_nw = 1;                                     // walker wavefronts per workgroup
     std::vector<int32_t> pairs_even, pairs_odd;
     DevBuf<int32_t> d_pairs_even, d_pairs_odd;
@@ -488,14 +501,29 @@ int tree_producers(int nw) { return nw <= 2 ? 2 : 4; }
 
 template <int MODEL>
 int launch_sweep_tree(rewl_ctx* c, int nsweeps) {
-    const int ng = (int)c->tree_groups[MODEL].size();
+    constexpr int list = 2 * MODEL;
+    const int ng = (int)c->tree_groups[list].size();
     if (ng == 0) return REWL_OK;
-    const size_t lds = c->tree_lds_bytes[MODEL];
+    const size_t lds = c->tree_lds_bytes[list];
     const int nw = c->tree_nw;
     HIP_TRY(hipFuncSetAttribute((const void*)k_sweep_tree<MODEL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k_sweep_tree<MODEL>, dim3((unsigned)ng), dim3((unsigned)(kLanes * (nw + tree_producers(nw)))), lds,
-                       c->stream, c->args, (const TreeScale*)c->d_tree_scale.p, (const int32_t*)c->d_tree_groups[MODEL].p,
+                       c->stream, c->args, (const TreeScale*)c->d_tree_scale.p, (const int32_t*)c->d_tree_groups[list].p,
                        ng, nsweeps, c->sweep_index, nw);
+    HIP_TRY(hipGetLastError());
+    return REWL_OK;
+}
+
+template <int MODEL>
+int launch_sweep_field_tree(rewl_ctx* c, int nsweeps) {
+    constexpr int list = 2 * MODEL + 1;
+    const int ng = (int)c->tree_groups[list].size();
+    if (ng == 0) return REWL_OK;
+    const size_t lds = c->tree_lds_bytes[list];
+    HIP_TRY(hipFuncSetAttribute((const void*)k_sweep_field_tree<MODEL>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds));
+    hipLaunchKernelGGL(k_sweep_field_tree<MODEL>, dim3((unsigned)ng), dim3(3 * kLanes), lds, c->stream, c->args,
+                       (const int32_t*)c->d_tree_groups[list].p, ng, nsweeps, c->sweep_index);
     HIP_TRY(hipGetLastError());
     return REWL_OK;
 }
@@ -559,6 +587,8 @@ int launch_sweeps(rewl_ctx* c, int nsweeps) {
     if ((rc = launch_tuned_all<1>(c, nsweeps))) return rc;
     if ((rc = launch_sweep_tree<0>(c, nsweeps))) return rc;
     if ((rc = launch_sweep_tree<1>(c, nsweeps))) return rc;
+    if ((rc = launch_sweep_field_tree<0>(c, nsweeps))) return rc;
+    if ((rc = launch_sweep_field_tree<1>(c, nsweeps))) return rc;
     HIP_TRY(hipEventRecord(e1, c->stream));
     c->ev_sweep.emplace_back(e0, e1);
     if (c->ev_sweep.size() > 256) return resolve_sweep_events(c);
@@ -714,7 +744,8 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
 
     // ---- systems swept with sixteen lanes a walker -------------------------------
     // When the caller asks for no particular kernel or launch shape and the
-    // context has few enough walkers (kTreeMaxWalkers).  One, two or four
+    // context has few enough walkers (kTreeMaxWalkers, kFieldTreeMaxWalkers).
+    // Integer energies: one, two or four
     // walker wavefronts (4, 8, 16 walkers) per workgroup, so that the
     // workgroups of a small context spread over the CUs (104 cycles an attempt
     // alone on a CU, 115 with a second walker wavefront, 137 with four), as far
@@ -747,6 +778,22 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         }
         for (size_t si = 0; si < c->sys.size(); ++si)
             if (tree_sys[si] && !fits(c->sys[si], c->tree_nw, &tree_scales[si])) tree_sys[si] = 0;
+        int64_t attempts = 0, largest = 1;   // of the FP64 systems, per sweep: all walkers', one walker's at most
+        for (const HostSystem& S : c->sys) {
+            if (S.intpath) continue;
+            attempts += (int64_t)S.ndof * S.d.num_windows * S.d.replicas_per_window;
+            largest = std::max<int64_t>(largest, S.ndof);
+        }
+        const bool few = attempts <= largest * kFieldTreeMaxWalkers;
+        for (size_t si = 0; shape_free && few && si < c->sys.size(); ++si) {
+            const HostSystem& S = c->sys[si];
+            if (S.intpath || S.d.L < kTreeMinL) continue;
+            int nb = 1;
+            for (int k = 0; k < S.d.num_windows; ++k) nb = std::max(nb, c->win[S.first_window + k].nbins);
+            if ((long long)nb * 12 * kTreePerWave > c->lds_max) continue;   // keeps the sum below in range
+            const ModelInfo m = model_info(S.d.model);
+            if (field_tree_lds(m.planes, m.energy_terms, S.d.L, nb).total <= c->lds_max) tree_sys[si] = 1;
+        }
     }
 
     // ---- wavefront groups -----------------------------------------------------
@@ -781,7 +828,8 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
             return bail(fail(REWL_ERR_INVALID, "the row-unrolled kernel needs the Philox integer path, producers >= 0 "
                                                "and L in {16, 24, 32, 48, 64}; with observables, sweep_kernel 0 or 3 "
                                                "and no densities"));
-        int wpg = tree ? c->tree_nw * kTreePerWave : kLanes;
+        const bool field_tree = tree && !S.intpath;
+        int wpg = field_tree ? kTreePerWave : tree ? c->tree_nw * kTreePerWave : kLanes;
         // guard bins: |Delta E| <= 4 (2J) (+ 4 (2K)) on the integer path
         int guard = 0;
         if (tuned) {
@@ -798,7 +846,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         else if (fast && !tree)
             wpg = std::min(kLanes, (int)((size_t)c->lds_max /
                                          ((size_t)(maxbins + 1) * 12 + (c->nprod ? 8 * (size_t)S.d.L : 0))));
-        else if (field_fast) {
+        else if (field_fast && !tree) {
             const long long room = (long long)c->lds_max - 16 - 8LL * S.N;
             wpg = room <= 0 ? 0 : std::min<long long>(kLanes, room / (12LL * maxbins + 16LL * S.d.L));
         } else if (P.observables == 2) {
@@ -843,11 +891,13 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
                 c->w_lat[g] = G.lat_base + j;
             }
             if (tree) {
-                c->tree_groups[S.d.model].push_back(gid);
+                const int list = 2 * S.d.model + (field_tree ? 1 : 0);
+                c->tree_groups[list].push_back(gid);
                 const TreeScale& t = tree_scales[(size_t)si];
-                c->tree_lds_bytes[S.d.model] =
-                    std::max(c->tree_lds_bytes[S.d.model],
-                             (size_t)tree_lds(planes, S.d.L, nb, c->tree_nw, t.pitch, t.guard).total);
+                const int terms = model_info(S.d.model).energy_terms;
+                const int bytes = field_tree ? field_tree_lds(planes, terms, S.d.L, nb).total
+                                             : tree_lds(planes, S.d.L, nb, c->tree_nw, t.pitch, t.guard).total;
+                c->tree_lds_bytes[list] = std::max(c->tree_lds_bytes[list], (size_t)bytes);
             } else if (tuned) {
                 c->tuned_groups[S.d.model][li].push_back(gid);
                 c->tuned_maxbins[S.d.model][li] = std::max(c->tuned_maxbins[S.d.model][li], nb);
@@ -956,7 +1006,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         std::stable_sort(list.begin(), list.end(), [&](int32_t x, int32_t y) {
             return c->sys[(size_t)c->groups[(size_t)x].sys].ndof > c->sys[(size_t)c->groups[(size_t)y].sys].ndof;
         });
-    for (int m = 0; m < 2; ++m)
+    for (int m = 0; m < 4; ++m)
         if ((rc = upload(c->d_tree_groups[m], c->tree_groups[m], c->stream))) return bail(rc);
     if ((rc = upload(c->d_tree_scale, tree_scales, c->stream))) return bail(rc);
     for (int cls = 0; cls < 4; ++cls)
@@ -990,7 +1040,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
     for (int cls = 0; cls < 4; ++cls) c->class_groups_all[cls] = c->class_groups[cls];
     for (int m = 0; m < 2; ++m)
         for (int i = 0; i < 5; ++i) c->tuned_groups_all[m][i] = c->tuned_groups[m][i];
-    for (int m = 0; m < 2; ++m) c->tree_groups_all[m] = c->tree_groups[m];
+    for (int m = 0; m < 4; ++m) c->tree_groups_all[m] = c->tree_groups[m];
     c->pairs_even_all = c->pairs_even;
     c->pairs_odd_all = c->pairs_odd;
     if ((rc = upload(c->d_w_flavor, flav, c->stream))) return bail(rc);
@@ -1192,7 +1242,7 @@ static int retire_done_systems(rewl_ctx* c) {
             keep(c->tuned_groups[m][i]);
             if ((rc = overwrite(c->d_tuned_groups[m][i], c->tuned_groups[m][i], c->stream))) return rc;
         }
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < 4; ++m) {
         keep(c->tree_groups[m]);
         if ((rc = overwrite(c->d_tree_groups[m], c->tree_groups[m], c->stream))) return rc;
     }
@@ -1228,7 +1278,7 @@ static int unretire_all(rewl_ctx* c) {
             c->tuned_groups[m][i] = c->tuned_groups_all[m][i];
             if ((rc = overwrite(c->d_tuned_groups[m][i], c->tuned_groups[m][i], c->stream))) return rc;
         }
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < 4; ++m) {
         c->tree_groups[m] = c->tree_groups_all[m];
         if ((rc = overwrite(c->d_tree_groups[m], c->tree_groups[m], c->stream))) return rc;
     }

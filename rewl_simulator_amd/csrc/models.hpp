@@ -66,15 +66,22 @@ struct Model<0> {
                                              const double nb[1][4]) {
         return E + (-0.5 * h * own[0] + 0.5 * local_energy(J, K, hf, h, own, nb));
     }
-    // E' of flipping the spin (change_state, ising2d_hamiltonian.hpp:216-222):
-    // E + (-1 t) f - (-1 s) f with t = -s
-    __device__ static double proposal_energy(double J, double, bool, double h, double E, const double own[1],
-                                             const double nb[1][4], int) {
+    // E' of flipping the spin is (E + a) + b (change_state,
+    // ising2d_hamiltonian.hpp:216-222): E + (-1 t) f - (-1 s) f with t = -s, so
+    // both terms are s f
+    static constexpr int kEnergyTerms = 1;   // distinct terms
+    __device__ static void energy_terms(double J, double, bool, double h, const double own[1], const double nb[1][4], int,
+                                        double& a, double& b) {
         double f = h;
 #pragma unroll
         for (int k = 0; k < 4; ++k) f = add_term(f, J, nb[0][k]);
-        const double sv = own[0], t = -sv;
-        return E + -1. * t * f - -1. * sv * f;
+        a = b = own[0] * f;
+    }
+    __device__ static double proposal_energy(double J, double K, bool hf, double h, double E, const double own[1],
+                                             const double nb[1][4], int fl) {
+        double a, b;
+        energy_terms(J, K, hf, h, own, nb, fl, a, b);
+        return (E + a) + b;
     }
 
     // Packed integer path.  One row's static slices: per site the count of
@@ -162,13 +169,14 @@ struct Model<1> {
         if (has_field) E += -0.5 * h * own[0] * own[1];
         return E + 0.5 * local_energy(J, K, has_field, h, own, nb);
     }
-    // E' of flipping sigma (fl = 0) or tau (fl = 1) of a site (change_state,
-    // ashkin_teller2d_hamiltonian.hpp:223-250): E + local(new) - local(old),
-    // each sum in the reference's order.  One of sigma, tau flips, so the
+    // E' of flipping sigma (fl = 0) or tau (fl = 1) of a site is (E + a) + b
+    // (change_state, ashkin_teller2d_hamiltonian.hpp:223-250): E + local(new) -
+    // local(old), each sum in the reference's order.  One of sigma, tau flips, so the
     // proposal's products K s t and h (s t) are the current ones negated,
     // exactly (every factor is +-1 or the coupling, a negation is exact).
-    __device__ static double proposal_energy(double J, double K, bool has_field, double h, double E,
-                                             const double own[2], const double nb[2][4], int fl) {
+    static constexpr int kEnergyTerms = 2;
+    __device__ static void energy_terms(double J, double K, bool has_field, double h, const double own[2],
+                                        const double nb[2][4], int fl, double& a, double& b) {
         const double sg = own[0], ta = own[1];
         const double Js = J * sg, Jt = J * ta, Kst = K * sg * ta;
         const double hst = has_field ? h * (sg * ta) : 0.;
@@ -185,7 +193,14 @@ struct Model<1> {
             en_old = add_term(en_old, Jt, nb[1][k]);
             en_old = add_term(en_old, Kst, nn);
         }
-        return E + -en_new - -en_old;
+        a = -en_new;
+        b = en_old;
+    }
+    __device__ static double proposal_energy(double J, double K, bool has_field, double h, double E,
+                                             const double own[2], const double nb[2][4], int fl) {
+        double a, b;
+        energy_terms(J, K, has_field, h, own, nb, fl, a, b);
+        return (E + a) + b;
     }
 
     // Packed integer path: the flipped plane P (and the other plane Q) give
@@ -273,13 +288,14 @@ struct Model<1> {
 struct ModelInfo {
     int planes, passes, values;
     bool product_coupling;
+    int energy_terms;
     long long (*energy_step)(long long, long long);
     long long (*ground_energy)(long long, long long, long long);
 };
 template <int M>
 constexpr ModelInfo model_info_of() {
     return ModelInfo{Model<M>::kPlanes, Model<M>::kPasses, Model<M>::kValues, Model<M>::kProductCoupling,
-                     &Model<M>::energy_step, &Model<M>::ground_energy};
+                     Model<M>::kEnergyTerms, &Model<M>::energy_step, &Model<M>::ground_energy};
 }
 inline ModelInfo model_info(int m) { return m == 0 ? model_info_of<0>() : model_info_of<1>(); }
 

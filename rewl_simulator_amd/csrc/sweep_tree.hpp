@@ -463,14 +463,15 @@ __device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGrou
 
 // Producer side: the bounds of the rows [r0, r0 + count) (rows of the launch,
 // counted over its passes and sweeps) for every walker of the group, one
-// Philox block (up to four bounds) per lane.
+// Philox block (up to four bounds) per lane.  A walker's ring of ringw bytes
+// holds `slots` rows of rowb bytes.
 template <int MODEL>
-__device__ __forceinline__ void tree_fill(const DevGroup& G, const DevSystem& S, const TreeLds& o, int ptid, int nthreads,
-                                          uint64_t sweep_base, int r0, int count, int nwpad, const BoundEntry* tab) {
+__device__ __forceinline__ void tree_fill(const DevGroup& G, const DevSystem& S, int ring, int ringw, int rowb, int slots,
+                                          int ptid, int nthreads, uint64_t sweep_base, int r0, int count, int nwpad,
+                                          const BoundEntry* tab) {
     const int L = S.L, per_sweep = Model<MODEL>::kPasses * L;
     const uint64_t blocks = (uint64_t)((S.ndof + 3) / 4);   // Philox blocks per sweep
     const int nbb = (L & 3) ? L / 4 + 2 : L / 4;            // blocks that a row can touch
-    const int seg2 = 2 * tree_seg_rows(L);
     const int total = count * nbb * nwpad;
     for (int i = ptid; i < total; i += nthreads) {
         const int j = i & (nwpad - 1);
@@ -488,7 +489,7 @@ __device__ __forceinline__ void tree_fill(const DevGroup& G, const DevSystem& S,
         const u32x4 w = philox4x32_10(u32x4{(uint32_t)bi, (uint32_t)(bi >> 32), DOMAIN_SWEEP, walker}, S.k0, S.k1);
         const double v[4] = {accept_bound(w.x, tab), accept_bound(w.y, tab), accept_bound(w.z, tab),
                              accept_bound(w.w, tab)};
-        const uint32_t dst = (uint32_t)(o.ring + j * o.ringw + (r % seg2) * L * 8);
+        const uint32_t dst = (uint32_t)(ring + j * ringw + (r % slots) * rowb);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int x = x0 + q;
@@ -541,11 +542,14 @@ __global__ void __launch_bounds__(512) k_sweep_tree(KArgs a, const TreeScale* sc
         } else {
             const int nrows = nsweeps * Mdl::kPasses * L, seg = tree_seg_rows(L);
             const int pt = tid - 64 * nw, pn = nth - 64 * nw;
-            tree_fill<MODEL>(G, S, o, pt, pn, sweep_base, 0, min(seg, nrows), SW, tab);
+            auto fill = [&](int r, int count) {
+                tree_fill<MODEL>(G, S, o.ring, o.ringw, 8 * L, 2 * seg, pt, pn, sweep_base, r, count, SW, tab);
+            };
+            fill(0, min(seg, nrows));
             __syncthreads();   // pairs with the walkers' barrier after the load
             for (int r = 0; r < nrows; r += seg) {
                 const int next = r + seg;
-                if (next < nrows) tree_fill<MODEL>(G, S, o, pt, pn, sweep_base, next, min(seg, nrows - next), SW, tab);
+                if (next < nrows) fill(next, min(seg, nrows - next));
                 __syncthreads();   // pairs with the walkers' end-of-segment barrier
             }
         }
