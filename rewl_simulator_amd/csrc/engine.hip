@@ -122,7 +122,10 @@ bool integral(double v) { return std::isfinite(v) && std::floor(v) == v && std::
 // Ising 104 / 161 at 512 walkers, 115 / 159 at 2048, 137 / 159 at 4096, 273 /
 // 159 at 5120; L = 32 Ashkin-Teller 128 / 198, 137 / 197, 155 / 197, 231 / 197.
 // Sizes without an unrolled-row kernel have the row kernel to compare with
-// (480-540 cycles): 215 at 8192, 389 at 12288.
+// (480-540 cycles): 215 at 8192, 389 at 12288.  With observables the sums take
+// the LDS of the walkers that would share a CU: L = 64 Ising with moments 313 /
+// 581 at 4096 and 576 / 572 at 5120, L = 20 Ashkin-Teller 828 / 1519 at 4096;
+// 4096 for every size.
 constexpr int kTreeMaxWalkers = 4096, kTreeMaxWalkersRow = 12288;
 // k_sweep_field_tree takes the FP64 systems of a context as long as their
 // walkers, each counted as its system's degrees of freedom over the largest
@@ -506,9 +509,11 @@ int launch_sweep_tree(rewl_ctx* c, int nsweeps) {
     if (ng == 0) return REWL_OK;
     const size_t lds = c->tree_lds_bytes[list];
     const int nw = c->tree_nw;
-    HIP_TRY(hipFuncSetAttribute((const void*)k_sweep_tree<MODEL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k_sweep_tree<MODEL>, dim3((unsigned)ng), dim3((unsigned)(kLanes * (nw + tree_producers(nw)))), lds,
-                       c->stream, c->args, (const TreeScale*)c->d_tree_scale.p, (const int32_t*)c->d_tree_groups[list].p,
+    void (*const kern)(KArgs, const TreeScale*, const int32_t*, int, int, uint64_t, int) =
+        c->p.observables == 2 ? k_sweep_tree<MODEL, 2> : c->p.observables ? k_sweep_tree<MODEL, 1> : k_sweep_tree<MODEL, 0>;
+    HIP_TRY(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, dim3((unsigned)ng), dim3((unsigned)(kLanes * (nw + tree_producers(nw)))), lds, c->stream,
+                       c->args, (const TreeScale*)c->d_tree_scale.p, (const int32_t*)c->d_tree_groups[list].p,
                        ng, nsweeps, c->sweep_index, nw);
     HIP_TRY(hipGetLastError());
     return REWL_OK;
@@ -753,8 +758,8 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
     std::vector<uint8_t> tree_sys(c->sys.size(), 0);
     std::vector<TreeScale> tree_scales(c->sys.size());
     {
-        const bool shape_free = P.rng_mode == REWL_RNG_PHILOX && P.observables == 0 && P.sweep_kernel == 0 &&
-                                P.producers == 0 && P.walkers_per_group == 0;
+        const bool shape_free = P.rng_mode == REWL_RNG_PHILOX && P.sweep_kernel == 0 && P.producers == 0 &&
+                                P.walkers_per_group == 0 && !P.densities;
         c->tree_nw = W <= 1024 ? 1 : W <= 2048 ? 2 : 4;
         auto fits = [&](const HostSystem& S, int nw, TreeScale* t) {
             if (!tree_scale(S.d, S.twoJ, S.twoK, nw, t)) return false;
@@ -762,12 +767,13 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
             for (int k = 0; k < S.d.num_windows; ++k) nb = std::max(nb, c->win[S.first_window + k].nbins);
             const long long bytes = (long long)(nb + 2 * t->guard) * t->pitch * 2;
             if (bytes > 4LL * c->lds_max) return false;   // keeps the sums below in range
-            return (size_t)tree_lds(model_info(S.d.model).planes, S.d.L, nb, nw, t->pitch, t->guard).total <=
+            const ModelInfo m = model_info(S.d.model);
+            return (size_t)tree_lds(m.planes, S.d.L, nb, nw, t->pitch, t->guard, P.observables, m.values).total <=
                    (size_t)c->lds_max;
         };
         for (size_t si = 0; shape_free && si < c->sys.size(); ++si) {
             const HostSystem& S = c->sys[si];
-            if (W > (tuned_index(S.d.L) >= 0 ? kTreeMaxWalkers : kTreeMaxWalkersRow)) continue;
+            if (W > (P.observables || tuned_index(S.d.L) >= 0 ? kTreeMaxWalkers : kTreeMaxWalkersRow)) continue;
             if (!S.intpath || S.d.L < kTreeMinL || !simple_range(S, c->win)) continue;
             TreeScale t;
             int nw = c->tree_nw;
@@ -785,7 +791,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
             largest = std::max<int64_t>(largest, S.ndof);
         }
         const bool few = attempts <= largest * kFieldTreeMaxWalkers;
-        for (size_t si = 0; shape_free && few && si < c->sys.size(); ++si) {
+        for (size_t si = 0; shape_free && !P.observables && few && si < c->sys.size(); ++si) {
             const HostSystem& S = c->sys[si];
             if (S.intpath || S.d.L < kTreeMinL) continue;
             int nb = 1;
@@ -849,7 +855,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         else if (field_fast && !tree) {
             const long long room = (long long)c->lds_max - 16 - 8LL * S.N;
             wpg = room <= 0 ? 0 : std::min<long long>(kLanes, room / (12LL * maxbins + 16LL * S.d.L));
-        } else if (P.observables == 2) {
+        } else if (!tree && P.observables == 2) {
             // ln g, counts and update counts per (bin, walker), plus the cos/sin table
             const long long room = (long long)c->lds_max - 16 - 16LL * S.d.L;
             wpg = room <= 0 ? 0 : std::min<long long>(kLanes, room / (16LL * maxbins));
@@ -896,7 +902,8 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
                 const TreeScale& t = tree_scales[(size_t)si];
                 const int terms = model_info(S.d.model).energy_terms;
                 const int bytes = field_tree ? field_tree_lds(planes, terms, S.d.L, nb).total
-                                             : tree_lds(planes, S.d.L, nb, c->tree_nw, t.pitch, t.guard).total;
+                                             : tree_lds(planes, S.d.L, nb, c->tree_nw, t.pitch, t.guard, P.observables,
+                                                        model_info(S.d.model).values).total;
                 c->tree_lds_bytes[list] = std::max(c->tree_lds_bytes[list], (size_t)bytes);
             } else if (tuned) {
                 c->tuned_groups[S.d.model][li].push_back(gid);

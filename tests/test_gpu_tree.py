@@ -83,3 +83,40 @@ def test_mixed_context(gpu):
     half = ising(9, 2, 3, 1.0, J=0.5, seed=3)
     half.update(e_min=-81.0, e_max=0.0)
     run_both([ising(16, 3, 2), ashkin_teller(11, 2, 5, seed=5), ising(24, 4, 3, 8.0, seed=7), half])
+
+
+@pytest.mark.parametrize("kernel", [{}, dict(producers=1)])
+@pytest.mark.parametrize("L", [5, 8, 13, 16, 30, 64])
+@pytest.mark.parametrize("obs", [1, 2])
+@pytest.mark.parametrize("model", ["ising", "at"])
+def test_observables(gpu, model, obs, L, kernel):
+    """The observable sums, and with 2 the correlator samples of a bin's
+    updates 0, 1000, 2000, ..., against the oracle's running means, over
+    several launches, exchanges and a check; chains and counts bit for bit."""
+    s = (ising(L, 3 if L < 20 else 12, 3, 8.0 if L > 40 else 4.0) if model == "ising" else
+         ashkin_teller(L, 3 if L < 20 else 24, 2))
+    p = configs.params(lnf_initial=0.05, observables=obs, sweeps_per_exchange=20, adjust_mode=1, **kernel)
+    # attempts for several samples of a bin where the oracle's time allows
+    per = max(2, 12000 // (L * L) // (1 if obs == 2 else 4))
+    with Engine([s], p) as eng:
+        ora = Oracle([s], p)
+        eng.adjust_to_range(); ora.adjust_to_range()
+        for k in range(4):
+            eng.sweeps(per); ora.sweeps(per)
+            eng.sweeps(1); ora.sweeps(1)
+            eng.exchange(); ora.exchange()
+            if k == 1:
+                eng.check(); ora.check()
+        assert_same(eng, ora, cursors=False)
+        corr = eng.correlator_slots(abi.ISING2D if model == "ising" else abi.ASHKIN_TELLER2D) if obs == 2 else []
+        for g in range(eng.num_walkers):
+            sums = eng.observables(g)
+            n = eng.counts(g).astype(np.float64) + eng.visits(g)
+            means, counts = ora.observables(g)
+            np.testing.assert_array_equal(n, counts, err_msg=f"counts per bin, walker {g}")
+            seen = n > 0
+            for c in range(sums.shape[1]):
+                div = np.ceil(n[seen] / 1000.0) if c in corr else n[seen]
+                np.testing.assert_allclose(sums[seen, c] / div, means[seen, c], rtol=1e-9, atol=1e-13,
+                                           err_msg=f"walker {g}, column {c}")
+            assert np.all(sums[~seen] == 0)
