@@ -115,18 +115,18 @@ std::vector<HostWindow> make_windows(const rewl_system_desc& d) {
 
 bool integral(double v) { return std::isfinite(v) && std::floor(v) == v && std::fabs(v) < 1e9; }
 
-// k_sweep_tree takes contexts of at most this many walkers: with 4096 its
-// workgroups (sixteen walkers, one per CU) fill the chip, and a second round of
-// them doubles its time per attempt while the kernels with one lane per walker
-// still have room.  Measured, cycles per attempt, tree against lane: L = 64
-// Ising 104 / 161 at 512 walkers, 115 / 159 at 2048, 137 / 159 at 4096, 273 /
-// 159 at 5120; L = 32 Ashkin-Teller 128 / 198, 137 / 197, 155 / 197, 231 / 197.
-// Sizes without an unrolled-row kernel have the row kernel to compare with
-// (480-540 cycles): 215 at 8192, 389 at 12288.  With observables the sums take
-// the LDS of the walkers that would share a CU: L = 64 Ising with moments 313 /
-// 581 at 4096 and 576 / 572 at 5120, L = 20 Ashkin-Teller 828 / 1519 at 4096;
-// 4096 for every size.
-constexpr int kTreeMaxWalkers = 4096, kTreeMaxWalkersRow = 12288;
+// k_sweep_tree takes contexts of at most this many walkers: 1280 workgroups of
+// four walkers, five per CU; beyond, its time per attempt grows with the walkers
+// while the kernels with one lane per walker still have room.  Measured, cycles
+// per attempt, tree against lane: L = 64 Ising 103 / 161 at 512 walkers, 110 /
+// 159 at 2048, 131 / 164 at 4096, 161 / 165 at 5120, 246 / 168 at 6144; L = 32
+// Ashkin-Teller 129 / 198, 141 / 198 at 4096, 184 / 198, 236 / 198.  Sizes
+// without an unrolled-row kernel have the row kernel to compare with (470-530
+// cycles): 225 at 8192.  With observables the sums take the LDS of the walkers
+// that would share a CU: with moments L = 64 Ising 348 / 564 at 4096, L = 16
+// Ashkin-Teller 641 / 845 at 4096 and 858 / 845 at 5120, L = 20 636 / 1513 and
+// 1338 / 1520.
+constexpr int kTreeMaxWalkers = 5120, kTreeMaxWalkersRow = 12288, kTreeMaxWalkersObs = 4096;
 // k_sweep_field_tree takes the FP64 systems of a context as long as their
 // walkers, each counted as its system's degrees of freedom over the largest
 // system's, are at most this many: 1024 workgroups, four per CU (registers and
@@ -196,7 +196,6 @@ struct rewl_ctx {
     DevBuf<int32_t> d_tree_groups[4];
     DevBuf<TreeScale> d_tree_scale;                      // per system
     size_t tree_lds_bytes[4] = {0, 0, 0, 0};             // the largest group's LDS
-    int tree_nw = 1;                                     // walker wavefronts per workgroup
     std::vector<int32_t> pairs_even, pairs_odd;
     DevBuf<int32_t> d_pairs_even, d_pairs_odd;
 
@@ -498,23 +497,18 @@ int launch_sweep_tuned(rewl_ctx* c, int li, int nsweeps) {
     return REWL_OK;
 }
 
-// Producer wavefronts of a k_sweep_tree workgroup: with one or two walker
-// wavefronts each of the four has a SIMD of its own.
-int tree_producers(int nw) { return nw <= 2 ? 2 : 4; }
-
 template <int MODEL>
 int launch_sweep_tree(rewl_ctx* c, int nsweeps) {
     constexpr int list = 2 * MODEL;
     const int ng = (int)c->tree_groups[list].size();
     if (ng == 0) return REWL_OK;
     const size_t lds = c->tree_lds_bytes[list];
-    const int nw = c->tree_nw;
-    void (*const kern)(KArgs, const TreeScale*, const int32_t*, int, int, uint64_t, int) =
+    void (*const kern)(KArgs, const TreeScale*, const int32_t*, int, int, uint64_t) =
         c->p.observables == 2 ? k_sweep_tree<MODEL, 2> : c->p.observables ? k_sweep_tree<MODEL, 1> : k_sweep_tree<MODEL, 0>;
     HIP_TRY(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3((unsigned)ng), dim3((unsigned)(kLanes * (nw + tree_producers(nw)))), lds, c->stream,
-                       c->args, (const TreeScale*)c->d_tree_scale.p, (const int32_t*)c->d_tree_groups[list].p,
-                       ng, nsweeps, c->sweep_index, nw);
+    hipLaunchKernelGGL(kern, dim3((unsigned)ng), dim3(2 * kLanes), lds, c->stream, c->args,
+                       (const TreeScale*)c->d_tree_scale.p, (const int32_t*)c->d_tree_groups[list].p, ng, nsweeps,
+                       c->sweep_index);
     HIP_TRY(hipGetLastError());
     return REWL_OK;
 }
@@ -600,11 +594,10 @@ int launch_sweeps(rewl_ctx* c, int nsweeps) {
     return REWL_OK;
 }
 
-// Byte scale of a system's states and energy changes in k_sweep_tree with `nw`
-// walker wavefronts per workgroup, and whether that kernel takes the system:
-// the state is energy x pitch / bin, stored energy changes are signed bytes
+// Byte scale of a system's states and energy changes in k_sweep_tree, and
+// whether that kernel takes the system: the state is energy x pitch / bin, stored energy changes are signed bytes
 // and their weight too.
-bool tree_scale(const rewl_system_desc& d, int twoJ, int twoK, int nw, TreeScale* out) {
+bool tree_scale(const rewl_system_desc& d, int twoJ, int twoK, TreeScale* out) {
     const bool kq = model_info(d.model).product_coupling;
     const long long bin = (long long)d.bin_size;
     if (bin < 1 || bin > 256) return false;
@@ -613,7 +606,7 @@ bool tree_scale(const rewl_system_desc& d, int twoJ, int twoK, int nw, TreeScale
     const long long g = std::gcd(2 * aJ, 2 * aK);   // energy changes: twoJ (4 - 2 k) + twoK (4 - 2 q)
     if (g == 0) return false;
     TreeScale t{};
-    const long long pitch = std::max<long long>(8 * kTreePerWave * nw, bin);
+    const long long pitch = std::max<long long>(8 * kTreePerWave, bin);
     const long long unit = pitch / bin * g;
     long long m = 1;
     while (unit / m > 127 && unit % (2 * m) == 0) m *= 2;
@@ -750,40 +743,28 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
     // ---- systems swept with sixteen lanes a walker -------------------------------
     // When the caller asks for no particular kernel or launch shape and the
     // context has few enough walkers (kTreeMaxWalkers, kFieldTreeMaxWalkers).
-    // Integer energies: one, two or four
-    // walker wavefronts (4, 8, 16 walkers) per workgroup, so that the
-    // workgroups of a small context spread over the CUs (104 cycles an attempt
-    // alone on a CU, 115 with a second walker wavefront, 137 with four), as far
-    // as the LDS of the widest window allows.
     std::vector<uint8_t> tree_sys(c->sys.size(), 0);
     std::vector<TreeScale> tree_scales(c->sys.size());
     {
         const bool shape_free = P.rng_mode == REWL_RNG_PHILOX && P.sweep_kernel == 0 && P.producers == 0 &&
                                 P.walkers_per_group == 0 && !P.densities;
-        c->tree_nw = W <= 1024 ? 1 : W <= 2048 ? 2 : 4;
-        auto fits = [&](const HostSystem& S, int nw, TreeScale* t) {
-            if (!tree_scale(S.d, S.twoJ, S.twoK, nw, t)) return false;
+        auto fits = [&](const HostSystem& S, TreeScale* t) {
+            if (!tree_scale(S.d, S.twoJ, S.twoK, t)) return false;
             int nb = 1;
             for (int k = 0; k < S.d.num_windows; ++k) nb = std::max(nb, c->win[S.first_window + k].nbins);
             const long long bytes = (long long)(nb + 2 * t->guard) * t->pitch * 2;
             if (bytes > 4LL * c->lds_max) return false;   // keeps the sums below in range
             const ModelInfo m = model_info(S.d.model);
-            return (size_t)tree_lds(m.planes, S.d.L, nb, nw, t->pitch, t->guard, P.observables, m.values).total <=
+            return (size_t)tree_lds(m.planes, S.d.L, nb, t->pitch, t->guard, P.observables, m.values).total <=
                    (size_t)c->lds_max;
         };
         for (size_t si = 0; shape_free && si < c->sys.size(); ++si) {
             const HostSystem& S = c->sys[si];
-            if (W > (P.observables || tuned_index(S.d.L) >= 0 ? kTreeMaxWalkers : kTreeMaxWalkersRow)) continue;
+            if (W > (P.observables ? kTreeMaxWalkersObs : tuned_index(S.d.L) >= 0 ? kTreeMaxWalkers : kTreeMaxWalkersRow))
+                continue;
             if (!S.intpath || S.d.L < kTreeMinL || !simple_range(S, c->win)) continue;
-            TreeScale t;
-            int nw = c->tree_nw;
-            while (nw >= 1 && !fits(S, nw, &t)) nw /= 2;
-            if (nw < 1) continue;
-            c->tree_nw = nw;
-            tree_sys[si] = 1;
+            if (fits(S, &tree_scales[si])) tree_sys[si] = 1;
         }
-        for (size_t si = 0; si < c->sys.size(); ++si)
-            if (tree_sys[si] && !fits(c->sys[si], c->tree_nw, &tree_scales[si])) tree_sys[si] = 0;
         int64_t attempts = 0, largest = 1;   // of the FP64 systems, per sweep: all walkers', one walker's at most
         for (const HostSystem& S : c->sys) {
             if (S.intpath) continue;
@@ -835,7 +816,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
                                                "and L in {16, 24, 32, 48, 64}; with observables, sweep_kernel 0 or 3 "
                                                "and no densities"));
         const bool field_tree = tree && !S.intpath;
-        int wpg = field_tree ? kTreePerWave : tree ? c->tree_nw * kTreePerWave : kLanes;
+        int wpg = tree ? kTreePerWave : kLanes;
         // guard bins: |Delta E| <= 4 (2J) (+ 4 (2K)) on the integer path
         int guard = 0;
         if (tuned) {
@@ -902,7 +883,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
                 const TreeScale& t = tree_scales[(size_t)si];
                 const int terms = model_info(S.d.model).energy_terms;
                 const int bytes = field_tree ? field_tree_lds(planes, terms, S.d.L, nb).total
-                                             : tree_lds(planes, S.d.L, nb, c->tree_nw, t.pitch, t.guard, P.observables,
+                                             : tree_lds(planes, S.d.L, nb, t.pitch, t.guard, P.observables,
                                                         model_info(S.d.model).values).total;
                 c->tree_lds_bytes[list] = std::max(c->tree_lds_bytes[list], (size_t)bytes);
             } else if (tuned) {

@@ -496,12 +496,13 @@ __device__ __forceinline__ void field_tree_terms(const DevGroup& G, const DevSys
 // One workgroup = one walker wavefront (four walkers) + two producers; groups
 // are taken persistently in blockIdx order.
 template <int MODEL>
-__global__ void __launch_bounds__(192, 3) k_sweep_field_tree(KArgs a, const int32_t* groups, int ngroups, int nsweeps,
-                                                          uint64_t sweep_base) {
+__global__ void __launch_bounds__(3 * kLanes, 3)
+    k_sweep_field_tree(KArgs a, const int32_t* groups, int ngroups, int nsweeps, uint64_t sweep_base) {
     using Mdl = Model<MODEL>;
     constexpr int NP = Mdl::kPlanes;
     constexpr int SW = kTreePerWave;
-    const int tid = threadIdx.x, nth = blockDim.x;
+    constexpr int nth = 3 * kLanes;
+    const int tid = threadIdx.x;
     const BoundEntry* tab = static_cast<const BoundEntry*>(a.bound_tab);
     if (tid < 64) __builtin_amdgcn_s_setprio(3);
     for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x) {
@@ -511,13 +512,30 @@ __global__ void __launch_bounds__(192, 3) k_sweep_field_tree(KArgs a, const int3
         const FieldTreeLds o = field_tree_lds(NP, Mdl::kEnergyTerms, L, G.nbins);
         // ---- load (LDS addresses are offsets: the kernel has no static LDS):
         // histograms, lattice; zeros where a row's last block has no site ------
-        for (int i = tid; i < (G.nbins + 1) * SW; i += nth) {
-            const int j = i & (SW - 1), b = i / SW;
-            const bool in = j < G.nwalkers && b < G.nbins;
-            const int64_t h = G.hist_base + j + (int64_t)b * kLanes;
-            const uint32_t at = (uint32_t)(o.hist + b * o.rowb);
-            lds_store_f64(at + 8u * (uint32_t)j, in ? a.lng[h] : __builtin_inf());
-            lds_store_u32(at + 8u * SW + 4u * (uint32_t)j, in ? a.cnt[h] : 0u);
+        // a thread loads one walker's bins, four at a time in flight
+        const int jw = tid & (SW - 1);
+        const bool there = jw < G.nwalkers;
+        const int64_t h0 = G.hist_base + jw;
+        constexpr int STEP = nth / SW;
+        for (int b0 = tid / SW; b0 <= G.nbins; b0 += 4 * STEP) {
+            double lng[4];
+            uint32_t cnt[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int b = b0 + k * STEP;
+                const bool in = there && b < G.nbins;
+                const int64_t h = h0 + (int64_t)b * kLanes;
+                lng[k] = in ? a.lng[h] : __builtin_inf();
+                cnt[k] = in ? a.cnt[h] : 0u;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int b = b0 + k * STEP;
+                if (b > G.nbins) continue;
+                const uint32_t at = (uint32_t)(o.hist + b * o.rowb);
+                lds_store_f64(at + 8u * (uint32_t)jw, lng[k]);
+                lds_store_u32(at + 8u * SW + 4u * (uint32_t)jw, cnt[k]);
+            }
         }
         for (int i = tid; i < NP * L * SW; i += nth) {
             const int j = i & (SW - 1), qy = i / SW;
@@ -540,7 +558,7 @@ __global__ void __launch_bounds__(192, 3) k_sweep_field_tree(KArgs a, const int3
                     h = field(r + 1);   // arrives before the next row needs it
                     field_tree_terms<MODEL>(G, S, o, lane, r, fl0, hr);
                 } else {
-                    tree_fill<MODEL>(G, S, o.ring, o.ringw, 32 * tree_blocks(L), 2, lane, kLanes, sweep_base, r, 1, SW, tab);
+                    tree_fill<MODEL>(G, S, o.ring, o.ringw, 32 * tree_blocks(L), 2, lane, sweep_base, r, 1, tab);
                 }
             };
             __syncthreads();   // LDS loaded
@@ -553,13 +571,11 @@ __global__ void __launch_bounds__(192, 3) k_sweep_field_tree(KArgs a, const int3
         }
         __syncthreads();   // the walkers' last updates are in LDS
         // ---- store -----------------------------------------------------------
-        for (int i = tid; i < G.nbins * SW; i += nth) {
-            const int j = i & (SW - 1), b = i / SW;
-            if (j >= G.nwalkers) continue;
-            const int64_t h = G.hist_base + j + (int64_t)b * kLanes;
+        for (int b = tid / SW; there && b < G.nbins; b += STEP) {
+            const int64_t h = h0 + (int64_t)b * kLanes;
             const uint32_t at = (uint32_t)(o.hist + b * o.rowb);
-            a.lng[h] = lds_f64(at + 8u * (uint32_t)j);
-            a.cnt[h] = lds_u32_at(at + 8u * SW + 4u * (uint32_t)j);
+            a.lng[h] = lds_f64(at + 8u * (uint32_t)jw);
+            a.cnt[h] = lds_u32_at(at + 8u * SW + 4u * (uint32_t)jw);
         }
         for (int i = tid; i < NP * L * SW; i += nth) {
             const int j = i & (SW - 1), qy = i / SW;

@@ -50,13 +50,15 @@
 // attempts.  Of the 440 cycles of a step the sixteen instructions of the
 // increments take 85, the FP64 atomic 50 and the count 25; a row adds 320.
 // Measured, cycles per attempt per walker, one lane a walker -> this kernel:
-// L = 64 Ising, 2048 walkers 158 -> 115 (270 -> 196 ms per 1000 sweeps); L = 16,
+// L = 64 Ising, 2048 walkers 158 -> 110 (270 -> 187 ms per 1000 sweeps); L = 16,
 // 8 walkers 253 -> 130; L = 42, 256 walkers (row kernel) 493 -> 112; L = 32
-// Ashkin-Teller, 512 walkers 196 -> 128.  Steps of three attempts cost 107 by
+// Ashkin-Teller, 512 walkers 196 -> 128.  A workgroup has one walker wavefront:
+// two (four) behind one barrier wait for each other and cost 114 at 2048 (137
+// at 4096) where one costs 110 (123); a second producer gained nothing.  Steps of three attempts cost 107 by
 // the same count and two 126.  With observables = 1, one lane a walker -> this
-// kernel: L = 64 Ising 273 -> 154 with 2048 walkers; L = 30 1012 -> 163; L = 32
-// Ashkin-Teller 798 -> 298.  With 2: L = 64 Ising 620 -> 212 (the samples 39 of
-// them, and 23 of 172 with 256 walkers), L = 30 2700 -> 191, Ashkin-Teller L = 32
+// kernel: L = 64 Ising 273 -> 157 with 2048 walkers; L = 30 1012 -> 163; L = 32
+// Ashkin-Teller 798 -> 298.  With 2: L = 64 Ising 620 -> 197 (the samples 23 of
+// 172 with 256 walkers), L = 30 2700 -> 191, Ashkin-Teller L = 32
 // 1256 -> 353, L = 20 4200 -> 381.  The spin flips as an LDS exclusive-or on the path
 // and the state hand-over before the updates measured no better.
 #pragma once
@@ -82,7 +84,7 @@ struct TreeScale {
     int32_t guard;   // guard bins on each side
 };
 
-// LDS of one workgroup of `nw` walker wavefronts (offsets in bytes).
+// LDS of one workgroup: four walkers (offsets in bytes).
 struct TreeLds {
     int32_t rowb, lat, ring, ringw, rec, queue, cnt, lng, sums, total;
 };
@@ -101,9 +103,8 @@ constexpr __host__ __device__ int tree_blocks(int L) { return (L + 3) / 4; }
 constexpr __host__ __device__ int tree_seg_rows(int L) { return L >= 32 ? 1 : (32 + L - 1) / L; }
 
 // `obs`: observables (0, 1, 2), `values` of them per update
-__host__ __device__ inline TreeLds tree_lds(int planes, int L, int nbins, int nw, int pitch, int guard, int obs,
-                                            int values) {
-    const int S = nw * kTreePerWave;
+__host__ __device__ inline TreeLds tree_lds(int planes, int L, int nbins, int pitch, int guard, int obs, int values) {
+    constexpr int S = kTreePerWave;
     TreeLds t;
     t.rowb = (tree_blocks(L) + 3) & ~3;                    // a row of nibbles
     t.lat = 0;                                             // [walker][plane][row]
@@ -111,7 +112,7 @@ __host__ __device__ inline TreeLds tree_lds(int planes, int L, int nbins, int nw
     t.ring = (t.lat + S * (planes * L * t.rowb + 4) + 15) & ~15;
     t.rec = t.ring + S * t.ringw;                          // [walker] kTreeRow bytes, see there
     t.queue = t.rec + S * (obs ? TreeRow<true>::kBytes : TreeRow<false>::kBytes);
-    const int other = t.queue + (obs == 2 ? nw * kTreePerWave * 4 * tree_blocks(L) * 8 : 0);
+    const int other = t.queue + (obs == 2 ? S * 4 * tree_blocks(L) * 8 : 0);
     const int nb = nbins + 2 * guard;
     // ln g at twice the offset of the counts, so that a count's address is
     // half its ln g's
@@ -421,8 +422,8 @@ __device__ __forceinline__ double tree_fourier(int L, int lane, uint64_t w, doub
 // state words hold the flips of its blocks.
 template <int MODEL>
 __device__ __forceinline__ void tree_samples(const KArgs& a, const DevGroup& G, const DevSystem& S, const TreeScale& T,
-                                          const TreeLds& o, int wave, int lane, int y, const TreeObs& ob, double co,
-                                          double si, int fl) {
+                                          const TreeLds& o, int lane, int y, const TreeObs& ob, double co, double si,
+                                          int fl) {
     using Mdl = Model<MODEL>;
     constexpr int NP = Mdl::kPlanes;
     using Row = TreeRow<true>;
@@ -431,8 +432,8 @@ __device__ __forceinline__ void tree_samples(const KArgs& a, const DevGroup& G, 
         const u32x2v e = lds_u32x2(ob.queue + 8u * k);
         const uint32_t slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)e.x);
         const uint32_t what = (uint32_t)__builtin_amdgcn_readfirstlane((int)e.y);
-        const int j = kTreePerWave * wave + (int)(what & 15u), block = (int)(what >> 8);
-        const int pf = Mdl::flip_plane(__builtin_amdgcn_readlane(fl, 16 * (int)(what & 3u)));
+        const int j = (int)(what & 15u), block = (int)(what >> 8);
+        const int pf = Mdl::flip_plane(__builtin_amdgcn_readlane(fl, 16 * j));
         const uint32_t words = (uint32_t)(o.rec + j * Row::kBytes + Row::kState + 4);
         uint64_t fw = (uint64_t)((what >> 4) & 15u) << (4 * block);
 #pragma unroll
@@ -464,10 +465,10 @@ __device__ __forceinline__ void tree_samples(const KArgs& a, const DevGroup& G, 
     }
 }
 
-// One walker wavefront: walkers 4 wave .. 4 wave + 3 of the group.
+// The walker wavefront: four walkers.
 template <int MODEL, int OBS>
 __device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGroup& G, const DevSystem& S,
-                                                   const TreeScale& T, const TreeLds& o, int wave, int nsweeps) {
+                                                   const TreeScale& T, const TreeLds& o, int nsweeps) {
     using Mdl = Model<MODEL>;
     constexpr int NP = Mdl::kPlanes;
     constexpr int NPASS = Mdl::kPasses;
@@ -475,8 +476,7 @@ __device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGrou
     using Row = TreeRow<OBS != 0>;
     constexpr uint32_t WB = Row::kWord;
     const int tid = threadIdx.x & 63;
-    const int n = tid & 15, row = tid >> 4;
-    const int j = kTreePerWave * wave + row;
+    const int n = tid & 15, j = tid >> 4;
     const bool active = j < G.nwalkers;
     const int g = G.first_walker + (active ? j : 0);
     const DevWindow Wn = a.win[a.w_window[g]];
@@ -516,10 +516,10 @@ __device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGrou
         c.f1 = t >= 2 ? lnf : 0.0;
         c.f2 = t >= 3 ? lnf : 0.0;
         c.f3 = t >= 1 ? lnf : 0.0;
-        const uint32_t sh = 16u * (row & 1);
+        const uint32_t sh = 16u * (j & 1);
         const bool on = active && n > 0;
-        c.mlo = on && row < 2 ? anc << sh : 0u;
-        c.mhi = on && row >= 2 ? anc << sh : 0u;
+        c.mlo = on && j < 2 ? anc << sh : 0u;
+        c.mhi = on && j >= 2 ? anc << sh : 0u;
         c.want = on ? want << sh : 0xffffffffu;
         c.want_tail = on && t < tail ? want << sh : 0xffffffffu;
         uint32_t flips = 0;
@@ -561,7 +561,7 @@ __device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGrou
     TreeState st{u0 + (uint32_t)(e0 << (pshift - bshift)), 0u, 0, 0};
     // an absent walker's row never writes its state words
     if (n < nblk) lds_store_u32x2(recw + (uint32_t)Row::kState + WB * (uint32_t)n, u32x2v{st.u, 0u});
-    TreeObs ob{L * L, 0, false, (uint32_t)(o.queue + wave * kTreePerWave * 4 * nblk * 8), 0u};
+    TreeObs ob{L * L, 0, false, (uint32_t)o.queue, 0u};
     // observables = 2: lane k has cos and sin of qmin k
     double co = 0.0, si = 0.0;
     if constexpr (OBS == 2) {
@@ -768,7 +768,7 @@ __device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGrou
         tree_block<MODEL, OBS, true, 0>(c, st, in, ob, 0u, 0u, mask, au_tail + WB * nlast,
                                         recw + WB * nlast + (uint32_t)Row::kState, nlast);
         if constexpr (OBS == 2) {
-            if (ob.due) tree_samples<MODEL>(a, G, S, T, o, wave, tid, y, ob, co, si, fl);
+            if (ob.due) tree_samples<MODEL>(a, G, S, T, o, tid, y, ob, co, si, fl);
         }
         up = own ^ (((last_block ? st.out : word) >> 4) & 15u);
         if (n < nblk) lds_store_u8(lat + (uint32_t)(y * o.rowb + n), up);
@@ -789,21 +789,20 @@ __device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGrou
     }
 }
 
-// Producer side: the bounds of the rows [r0, r0 + count) (rows of the launch,
-// counted over its passes and sweeps) for every walker of the group, one
-// Philox block (up to four bounds) per lane.  A walker's ring of ringw bytes
+// Producer side, one wavefront: the bounds of the rows [r0, r0 + count) (rows of
+// the launch, counted over its passes and sweeps) for every walker of the
+// group, one Philox block (up to four bounds) per lane.  A walker's ring of ringw bytes
 // holds `slots` rows of rowb bytes.
 template <int MODEL>
 __device__ __forceinline__ void tree_fill(const DevGroup& G, const DevSystem& S, int ring, int ringw, int rowb, int slots,
-                                          int ptid, int nthreads, uint64_t sweep_base, int r0, int count, int nwpad,
-                                          const BoundEntry* tab) {
+                                          int lane, uint64_t sweep_base, int r0, int count, const BoundEntry* tab) {
     const int L = S.L, per_sweep = Model<MODEL>::kPasses * L;
     const uint64_t blocks = (uint64_t)((S.ndof + 3) / 4);   // Philox blocks per sweep
     const int nbb = (L & 3) ? L / 4 + 2 : L / 4;            // blocks that a row can touch
-    const int total = count * nbb * nwpad;
-    for (int i = ptid; i < total; i += nthreads) {
-        const int j = i & (nwpad - 1);
-        const int rest = i / nwpad;
+    const int total = count * nbb * kTreePerWave;
+    for (int i = lane; i < total; i += kLanes) {
+        const int j = i & (kTreePerWave - 1);
+        const int rest = i / kTreePerWave;
         const int k = rest / nbb, bb = rest - k * nbb;
         if (j >= G.nwalkers) continue;
         const int r = r0 + k;
@@ -826,34 +825,51 @@ __device__ __forceinline__ void tree_fill(const DevGroup& G, const DevSystem& S,
     }
 }
 
-// One workgroup = nw walker wavefronts (four walkers each) + producer
-// wavefronts; groups are taken persistently in blockIdx order.
+// One workgroup = one walker wavefront (four walkers) + one producer; groups
+// are taken persistently in blockIdx order.
 template <int MODEL, int OBS>
-__global__ void __launch_bounds__(512) k_sweep_tree(KArgs a, const TreeScale* scale, const int32_t* groups, int ngroups,
-                                                    int nsweeps, uint64_t sweep_base, int nw) {
+__global__ void __launch_bounds__(2 * kLanes) k_sweep_tree(KArgs a, const TreeScale* scale, const int32_t* groups,
+                                                           int ngroups, int nsweeps, uint64_t sweep_base) {
     using Mdl = Model<MODEL>;
     constexpr int NP = Mdl::kPlanes;
-    const int tid = threadIdx.x, nth = blockDim.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int SW = nw * kTreePerWave;
+    constexpr int SW = kTreePerWave;
+    constexpr int nth = 2 * kLanes;
+    const int tid = threadIdx.x;
+    const bool walkers = __builtin_amdgcn_readfirstlane(tid) < kLanes;
     const BoundEntry* tab = static_cast<const BoundEntry*>(a.bound_tab);
-    if (wave < nw) __builtin_amdgcn_s_setprio(3);
+    if (walkers) __builtin_amdgcn_s_setprio(3);
     for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x) {
         const DevGroup G = a.grp[groups[gi]];
         const DevSystem S = a.sys[G.sys];
         const TreeScale T = scale[G.sys];
         const int L = S.L;
-        const TreeLds o = tree_lds(NP, L, G.nbins, nw, T.pitch, T.guard, OBS, Mdl::kValues);
+        const TreeLds o = tree_lds(NP, L, G.nbins, T.pitch, T.guard, OBS, Mdl::kValues);
         // ---- load (LDS addresses are offsets: the kernel has no static LDS):
         // histograms (guard bins and absent walkers: +inf), lattice --
         const int nb = G.nbins + 2 * T.guard;
-        for (int i = tid; i < nb * SW; i += nth) {
-            const int j = i & (SW - 1), b = i / SW - T.guard;
-            const bool in = j < G.nwalkers && b >= 0 && b < a.win[a.w_window[G.first_walker + (j < G.nwalkers ? j : 0)]].nbins;
-            const int64_t h = G.hist_base + j + (int64_t)b * kLanes;
-            const uint32_t at = (uint32_t)((b + T.guard) * T.pitch + j * 8);
-            lds_store_f64((uint32_t)o.lng + at, in ? a.lng[h] : __builtin_inf());
-            lds_store_u32((uint32_t)o.cnt + at / 2, !in ? 0u : OBS == 2 ? cycle_word(a.obs_tot[h]) : a.cnt[h]);
+        // a thread loads one walker's bins, eight at a time in flight
+        const int jw = tid & (SW - 1), bins = jw < G.nwalkers ? a.win[a.w_window[G.first_walker + jw]].nbins : 0;
+        const int64_t h0 = G.hist_base + jw;
+        constexpr int STEP = nth / SW;
+        for (int b0 = tid / SW; b0 < nb; b0 += 8 * STEP) {
+            double lng[8];
+            uint32_t cnt[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int b = b0 + k * STEP - T.guard;
+                const bool in = b >= 0 && b < bins;
+                const int64_t h = h0 + (int64_t)b * kLanes;
+                lng[k] = in ? a.lng[h] : __builtin_inf();
+                cnt[k] = !in ? 0u : OBS == 2 ? a.obs_tot[h] : a.cnt[h];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int b = b0 + k * STEP;
+                if (b >= nb) continue;
+                const uint32_t at = (uint32_t)(b * T.pitch + jw * 8);
+                lds_store_f64((uint32_t)o.lng + at, lng[k]);
+                lds_store_u32((uint32_t)o.cnt + at / 2, OBS == 2 ? cycle_word(cnt[k]) : cnt[k]);
+            }
         }
         if constexpr (OBS != 0)
             for (int i = tid; i < (o.total - o.sums) / 8; i += nth) lds_store_f64((uint32_t)(o.sums + 8 * i), 0.0);
@@ -867,13 +883,12 @@ __global__ void __launch_bounds__(512) k_sweep_tree(KArgs a, const TreeScale* sc
                               (x & 0xfu) | ((x & 0xf0u) << 4) | ((x & 0xf00u) << 8) | ((x & 0xf000u) << 12));
             }
         }
-        if (wave < nw) {
-            sweep_walkers_tree<MODEL, OBS>(a, G, S, T, o, wave, nsweeps);
+        if (walkers) {
+            sweep_walkers_tree<MODEL, OBS>(a, G, S, T, o, nsweeps);
         } else {
             const int nrows = nsweeps * Mdl::kPasses * L, seg = tree_seg_rows(L);
-            const int pt = tid - 64 * nw, pn = nth - 64 * nw;
             auto fill = [&](int r, int count) {
-                tree_fill<MODEL>(G, S, o.ring, o.ringw, 8 * L, 2 * seg, pt, pn, sweep_base, r, count, SW, tab);
+                tree_fill<MODEL>(G, S, o.ring, o.ringw, 8 * L, 2 * seg, tid - kLanes, sweep_base, r, count, tab);
             };
             fill(0, min(seg, nrows));
             __syncthreads();   // pairs with the walkers' barrier after the load
@@ -885,11 +900,9 @@ __global__ void __launch_bounds__(512) k_sweep_tree(KArgs a, const TreeScale* sc
         }
         __syncthreads();   // the walkers' last updates are in LDS
         // ---- store -----------------------------------------------------------
-        for (int i = tid; i < G.nbins * SW; i += nth) {
-            const int j = i & (SW - 1), b = i / SW;
-            if (j >= G.nwalkers || b >= a.win[a.w_window[G.first_walker + j]].nbins) continue;
-            const int64_t h = G.hist_base + j + (int64_t)b * kLanes;
-            const uint32_t at = (uint32_t)((b + T.guard) * T.pitch + j * 8);
+        for (int b = tid / SW; b < bins; b += STEP) {
+            const int64_t h = h0 + (int64_t)b * kLanes;
+            const uint32_t at = (uint32_t)((b + T.guard) * T.pitch + jw * 8);
             a.lng[h] = lds_f64((uint32_t)o.lng + at);
             const uint32_t cw = lds_u32_at((uint32_t)o.cnt + at / 2);
             if constexpr (OBS == 2) {
@@ -902,11 +915,11 @@ __global__ void __launch_bounds__(512) k_sweep_tree(KArgs a, const TreeScale* sc
             if constexpr (OBS != 0) {
                 // sums of bins without an update are zero
                 double* p = a.obs + h * a.nobs;
-                const uint32_t sum = (uint32_t)(o.sums + (b * T.pitch + j * 8) * Mdl::kValues);
+                const uint32_t sum = (uint32_t)(o.sums + (b * T.pitch + jw * 8) * Mdl::kValues);
 #pragma unroll
                 for (int k = 0; k < Mdl::kValues; ++k) {
                     const double v = lds_f64(sum + 8u * (uint32_t)k);
-                    if (v != 0.0) p[(k / 3) * (OBS == 2 ? 4 : 3) + k % 3] += v;
+                    if (v != 0.0) obs_add(p + (k / 3) * (OBS == 2 ? 4 : 3) + k % 3, v);
                 }
             }
         }
