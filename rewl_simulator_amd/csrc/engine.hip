@@ -237,6 +237,7 @@ struct rewl_ctx {
     int flush_every = 1;
     uint64_t sweep_index = 0;
     int64_t pending_sweeps = 0;
+    int exchange_waves = 1;   // of a k_exchange workgroup: the most replicas of a window, at most sixteen
     bool direction_even = true;
     bool in_windows = false;   // every walker inside its window (rewl_adjust_to_range ran)
     bool refining = false;     // between rewl_refine_begin and rewl_refine_end
@@ -729,6 +730,8 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         c->sys.push_back(std::move(S));
     }
     c->num_walkers = walker;
+    for (const HostSystem& S : c->sys)
+        c->exchange_waves = std::max(c->exchange_waves, std::min<int>(S.d.replicas_per_window, 16));
     const int W = walker;
 
     // ---- device limits ------------------------------------------------------
@@ -1192,7 +1195,7 @@ int rewl_exchange(rewl_ctx* c) {
     const std::vector<int32_t>& pl = even ? c->pairs_even : c->pairs_odd;
     if (!pl.empty()) {
         const int32_t* dp = even ? c->d_pairs_even.p : c->d_pairs_odd.p;
-        hipLaunchKernelGGL(k_exchange, dim3((unsigned)pl.size()), dim3(kLanes), 0, c->stream, c->args, dp,
+        hipLaunchKernelGGL(k_exchange, dim3((unsigned)pl.size()), dim3((unsigned)(kLanes * c->exchange_waves)), 0, c->stream, c->args, dp,
                            (int)pl.size(), c->p.rng_mode == REWL_RNG_REPLAY ? 1 : 0);
         HIP_TRY(hipGetLastError());
     }
