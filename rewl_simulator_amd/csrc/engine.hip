@@ -231,6 +231,7 @@ struct rewl_ctx {
     std::vector<std::mt19937_64> engines;
     std::vector<uint64_t> filled;
     uint64_t ring_cap = 0;
+    uint64_t replay_left = 0;   // every stream holds at least this many words not consumed
 
     hipStream_t stream = nullptr;
     int lds_max = 65536;
@@ -379,31 +380,43 @@ int clear_err_bits(rewl_ctx* c, int32_t bits) {
     return REWL_OK;
 }
 
-// Make sure every replay stream holds at least ring_cap unconsumed words.
-int replay_topup(rewl_ctx* c) {
+// Make sure every replay stream holds the `need` words that the next launch
+// can consume at most.  The cursors are read, and the streams filled up, only
+// when what earlier launches can have consumed leaves fewer (replay_left): with
+// a read, a copy per walker and a wait for each, a fill takes longer than the
+// five sweeps of an L = 12 launch.
+int replay_topup(rewl_ctx* c, uint64_t need) {
     if (c->p.rng_mode != REWL_RNG_REPLAY) return REWL_OK;
+    if (c->replay_left >= need) {
+        c->replay_left -= need;
+        return REWL_OK;
+    }
     const int W = c->num_walkers;
     std::vector<uint64_t> cur((size_t)W);
     HIP_TRY(hipMemcpyAsync(cur.data(), c->d_w_cursor.p, (size_t)W * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     const uint64_t C = c->ring_cap;
-    std::vector<uint64_t> tmp;
+    uint64_t words = 0;
+    for (int g = 0; g < W; ++g) words += cur[g] + C - std::min(cur[g] + C, c->filled[g]);
+    std::vector<uint64_t> tmp(words);
+    uint64_t* t = tmp.data();
     for (int g = 0; g < W; ++g) {
         const uint64_t target = cur[g] + C;
         uint64_t& f = c->filled[g];
         while (f < target) {
             const uint64_t pos = f & (C - 1);
             const uint64_t len = std::min<uint64_t>(target - f, C - pos);
-            tmp.resize(len);
-            for (uint64_t k = 0; k < len; ++k) tmp[k] = c->engines[g]();
-            HIP_TRY(hipMemcpyAsync(c->d_ring.p + (size_t)g * C + pos, tmp.data(), len * sizeof(uint64_t),
-                                   hipMemcpyHostToDevice, c->stream));
-            HIP_TRY(hipStreamSynchronize(c->stream));
+            for (uint64_t k = 0; k < len; ++k) t[k] = c->engines[g]();
+            HIP_TRY(hipMemcpyAsync(c->d_ring.p + (size_t)g * C + pos, t, len * sizeof(uint64_t), hipMemcpyHostToDevice,
+                                   c->stream));
+            t += len;
             f += len;
         }
     }
     HIP_TRY(hipMemcpyAsync(c->d_ring_filled.p, c->filled.data(), (size_t)W * sizeof(uint64_t), hipMemcpyHostToDevice,
                            c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));   // tmp goes
+    c->replay_left = C - std::min(need, C);
     return REWL_OK;
 }
 
@@ -1142,7 +1155,7 @@ int rewl_adjust_to_range(rewl_ctx* c) {
     // a failed earlier adjustment left the range bit set; it describes that
     // attempt only (the replay-exhausted bit stays: the streams are spent)
     if ((rc = clear_err_bits(c, 2))) return rc;
-    if ((rc = replay_topup(c))) return rc;
+    if ((rc = replay_topup(c, 1))) return rc;
     uint64_t steps = (uint64_t)max_ndof(c) * 4096ull;
     const int mode = c->p.adjust_mode;
     if (c->p.rng_mode == REWL_RNG_REPLAY)
@@ -1169,7 +1182,7 @@ int rewl_sweeps(rewl_ctx* c, int32_t n) {
                           : n;
     while (done < n) {
         const int k = std::min(chunk, n - done);
-        if ((rc = replay_topup(c))) return rc;
+        if ((rc = replay_topup(c, (uint64_t)k * (uint64_t)max_ndof(c)))) return rc;
         if ((rc = launch_sweeps(c, k))) return rc;
         c->sweep_index += (uint64_t)k;
         done += k;
@@ -1190,7 +1203,9 @@ int rewl_sweeps(rewl_ctx* c, int32_t n) {
 int rewl_exchange(rewl_ctx* c) {
     if (!c) return fail(REWL_ERR_INVALID, "null context");
     int rc;
-    if ((rc = replay_topup(c))) return rc;
+    // a draw per swap pair of the shuffle (at most kMaxReplicas / 2, rejections
+    // are one in 2^48) and one for the decision
+    if ((rc = replay_topup(c, kMaxReplicas))) return rc;
     const bool even = c->direction_even;
     const std::vector<int32_t>& pl = even ? c->pairs_even : c->pairs_odd;
     if (!pl.empty()) {
