@@ -69,6 +69,8 @@ __device__ __forceinline__ bool exp_less(double u, double x) {
     if (x == 0.) return u < 1.;
     if (u == 0.) return x > -745.1332191019412;   // RN(exp(x)) > 0
     if (x < -23.) return false;                   // exp(x) < 2^-33 <= u
+    const int told = against_exp(u, x);
+    if (told != 0) return told > 0;
     const double p = exp(x);
     if (u < p * (1. - 0x1p-48)) return true;
     if (u > p * (1. + 0x1p-48)) return false;

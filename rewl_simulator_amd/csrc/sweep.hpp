@@ -77,7 +77,8 @@ __device__ __forceinline__ bool wl_accept_int(int En, int& E, int& cb, double& l
     bool acc = in && (d <= 0.f);
     if (in && !(d <= 0.f)) {
         const double u = draw_uniform<REPLAY>(ring, cap, filled, cursor, err, rnd, p);
-        acc = u < exp(-(double)d);
+        const int told = against_exp(u, -(double)d);
+        acc = told > 0 || (told == 0 && u < exp(-(double)d));
     }
     if (acc) { E = En; cb = nb; lc = ln; }
     lc += lnf;
@@ -104,7 +105,8 @@ __device__ __forceinline__ bool wl_accept_fp(double En, double& E, int& cb, doub
     bool acc = in && (d <= 0.f);
     if (in && !(d <= 0.f)) {
         const double u = draw_uniform<REPLAY>(ring, cap, filled, cursor, err, rnd, p);
-        acc = u < exp(-(double)d);
+        const int told = against_exp(u, -(double)d);
+        acc = told > 0 || (told == 0 && u < exp(-(double)d));
     }
     if (acc) { E = En; cb = nb; lc = ln; }
     lc += lnf;
