@@ -6,6 +6,7 @@
 // device with four kinds of launch that replace the reference's per-rank loop
 // and its MPI traffic: sweep (one lane per walker), exchange (one wavefront
 // per adjacent window pair), check (one wavefront per window) and finalize.
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -245,6 +246,7 @@ struct rewl_ctx {
     int64_t refine_since_exchange = 0;
     rewl_stats stats{};
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_sweep;
+    std::vector<hipEvent_t> ev_free;   // at most as many as ev_sweep has held: 2 x 257
     std::vector<int32_t> done_host;
     KArgs args{};
 };
@@ -255,6 +257,8 @@ void destroy_ctx(rewl_ctx* c) {
     if (!c) return;
     for (auto& e : c->ev_sweep) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
     c->ev_sweep.clear();
+    for (auto& e : c->ev_free) (void)hipEventDestroy(e);
+    c->ev_free.clear();
     for (auto* b : {&c->d_w_window, &c->d_w_local, &c->d_w_flavor, &c->d_err, &c->d_win_oot, &c->d_win_done,
                     &c->d_win_active,
                     &c->d_pairs_even, &c->d_pairs_odd})
@@ -353,8 +357,8 @@ int resolve_sweep_events(rewl_ctx* c) {
         HIP_TRY(hipEventElapsedTime(&ms, e.first, e.second));
         c->stats.kernel_ms_sweep += ms;
         c->stats.sweep_launches += 1;
-        (void)hipEventDestroy(e.first);
-        (void)hipEventDestroy(e.second);
+        c->ev_free.push_back(e.first);
+        c->ev_free.push_back(e.second);
     }
     c->ev_sweep.clear();
     return REWL_OK;
@@ -511,8 +515,26 @@ int launch_sweep_tuned(rewl_ctx* c, int li, int nsweeps) {
     return REWL_OK;
 }
 
+// Events around a launch of sweeps (stats: kernel_ms_sweep), taken from a
+// pool.  Recorded by themselves they are packets of their own before and after
+// the kernel; when the launch is one kernel they ride on it.
+struct SweepEvents {
+    hipEvent_t start, stop;
+    bool one_kernel;
+};
+
+int take_event(rewl_ctx* c, hipEvent_t* e) {
+    if (c->ev_free.empty()) {
+        HIP_TRY(hipEventCreate(e));
+        return REWL_OK;
+    }
+    *e = c->ev_free.back();
+    c->ev_free.pop_back();
+    return REWL_OK;
+}
+
 template <int MODEL>
-int launch_sweep_tree(rewl_ctx* c, int nsweeps) {
+int launch_sweep_tree(rewl_ctx* c, int nsweeps, const SweepEvents& ev) {
     constexpr int list = 2 * MODEL;
     const int ng = (int)c->tree_groups[list].size();
     if (ng == 0) return REWL_OK;
@@ -520,23 +542,33 @@ int launch_sweep_tree(rewl_ctx* c, int nsweeps) {
     void (*const kern)(KArgs, const TreeScale*, const int32_t*, int, int, uint64_t) =
         c->p.observables == 2 ? k_sweep_tree<MODEL, 2> : c->p.observables ? k_sweep_tree<MODEL, 1> : k_sweep_tree<MODEL, 0>;
     HIP_TRY(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3((unsigned)ng), dim3(2 * kLanes), lds, c->stream, c->args,
-                       (const TreeScale*)c->d_tree_scale.p, (const int32_t*)c->d_tree_groups[list].p, ng, nsweeps,
-                       c->sweep_index);
+    KArgs args = c->args;
+    const TreeScale* scale = c->d_tree_scale.p;
+    const int32_t* gl = c->d_tree_groups[list].p;
+    int ngroups = ng;
+    uint64_t base = c->sweep_index;
+    void* kargs[] = {&args, (void*)&scale, (void*)&gl, &ngroups, &nsweeps, &base};
+    HIP_TRY(hipExtLaunchKernel((const void*)kern, dim3((unsigned)ng), dim3(2 * kLanes), kargs, lds, c->stream,
+                               ev.one_kernel ? ev.start : nullptr, ev.one_kernel ? ev.stop : nullptr, 0));
     HIP_TRY(hipGetLastError());
     return REWL_OK;
 }
 
 template <int MODEL>
-int launch_sweep_field_tree(rewl_ctx* c, int nsweeps) {
+int launch_sweep_field_tree(rewl_ctx* c, int nsweeps, const SweepEvents& ev) {
     constexpr int list = 2 * MODEL + 1;
     const int ng = (int)c->tree_groups[list].size();
     if (ng == 0) return REWL_OK;
     const size_t lds = c->tree_lds_bytes[list];
     HIP_TRY(hipFuncSetAttribute((const void*)k_sweep_field_tree<MODEL>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds));
-    hipLaunchKernelGGL(k_sweep_field_tree<MODEL>, dim3((unsigned)ng), dim3(3 * kLanes), lds, c->stream, c->args,
-                       (const int32_t*)c->d_tree_groups[list].p, ng, nsweeps, c->sweep_index);
+    KArgs args = c->args;
+    const int32_t* gl = c->d_tree_groups[list].p;
+    int ngroups = ng;
+    uint64_t base = c->sweep_index;
+    void* kargs[] = {&args, (void*)&gl, &ngroups, &nsweeps, &base};
+    HIP_TRY(hipExtLaunchKernel((const void*)k_sweep_field_tree<MODEL>, dim3((unsigned)ng), dim3(3 * kLanes), kargs, lds,
+                               c->stream, ev.one_kernel ? ev.start : nullptr, ev.one_kernel ? ev.stop : nullptr, 0));
     HIP_TRY(hipGetLastError());
     return REWL_OK;
 }
@@ -586,31 +618,47 @@ int launch_sweep_class(rewl_ctx* c, int cls, int nsweeps) {
     return REWL_OK;
 }
 
-int launch_sweeps(rewl_ctx* c, int nsweeps) {
-    hipEvent_t e0, e1;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    HIP_TRY(hipEventRecord(e0, c->stream));
+int launch_sweep_kernels(rewl_ctx* c, int nsweeps, SweepEvents& ev) {
     int rc;
+    int others = 0, trees = 0;
+    for (const auto& l : c->class_groups) others += l.empty() ? 0 : 1;
+    for (const auto& m : c->tuned_groups)
+        for (const auto& l : m) others += l.empty() ? 0 : 1;
+    for (const auto& l : c->tree_groups) trees += l.empty() ? 0 : 1;
+    ev.one_kernel = others == 0 && trees == 1;
+    if (!ev.one_kernel) HIP_TRY(hipEventRecord(ev.start, c->stream));
     if ((rc = launch_sweep_class<0, false>(c, 0, nsweeps))) return rc;
     if ((rc = launch_sweep_class<0, true>(c, 1, nsweeps))) return rc;
     if ((rc = launch_sweep_class<1, false>(c, 2, nsweeps))) return rc;
     if ((rc = launch_sweep_class<1, true>(c, 3, nsweeps))) return rc;
     if ((rc = launch_tuned_all<0>(c, nsweeps))) return rc;
     if ((rc = launch_tuned_all<1>(c, nsweeps))) return rc;
-    if ((rc = launch_sweep_tree<0>(c, nsweeps))) return rc;
-    if ((rc = launch_sweep_tree<1>(c, nsweeps))) return rc;
-    if ((rc = launch_sweep_field_tree<0>(c, nsweeps))) return rc;
-    if ((rc = launch_sweep_field_tree<1>(c, nsweeps))) return rc;
-    HIP_TRY(hipEventRecord(e1, c->stream));
-    c->ev_sweep.emplace_back(e0, e1);
+    if ((rc = launch_sweep_tree<0>(c, nsweeps, ev))) return rc;
+    if ((rc = launch_sweep_tree<1>(c, nsweeps, ev))) return rc;
+    if ((rc = launch_sweep_field_tree<0>(c, nsweeps, ev))) return rc;
+    if ((rc = launch_sweep_field_tree<1>(c, nsweeps, ev))) return rc;
+    if (!ev.one_kernel) HIP_TRY(hipEventRecord(ev.stop, c->stream));
+    return REWL_OK;
+}
+
+int launch_sweeps(rewl_ctx* c, int nsweeps) {
+    SweepEvents ev{};
+    int rc = take_event(c, &ev.start);
+    if (rc == REWL_OK) rc = take_event(c, &ev.stop);
+    if (rc == REWL_OK) rc = launch_sweep_kernels(c, nsweeps, ev);
+    if (rc != REWL_OK) {
+        if (ev.start) c->ev_free.push_back(ev.start);
+        if (ev.stop) c->ev_free.push_back(ev.stop);
+        return rc;
+    }
+    c->ev_sweep.emplace_back(ev.start, ev.stop);
     if (c->ev_sweep.size() > 256) return resolve_sweep_events(c);
     return REWL_OK;
 }
 
 // Byte scale of a system's states and energy changes in k_sweep_tree, and
-// whether that kernel takes the system: the state is energy x pitch / bin, stored energy changes are signed bytes
-// and their weight too.
+// whether that kernel takes the system: the state is energy x pitch / bin,
+// stored energy changes are signed bytes and their weight too.
 bool tree_scale(const rewl_system_desc& d, int twoJ, int twoK, TreeScale* out) {
     const bool kq = model_info(d.model).product_coupling;
     const long long bin = (long long)d.bin_size;
