@@ -905,6 +905,12 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
             const long long room = (long long)c->lds_max - 16 - 16LL * S.d.L;
             wpg = room <= 0 ? 0 : std::min<long long>(kLanes, room / (16LL * maxbins));
         }
+        // a system's windows are accepted or refused whichever kernel takes them
+        // (the walkers of the context decide that): with moments, off the
+        // unrolled-row sizes, those that the generic kernel holds
+        if (tree && P.observables == 1 && li < 0 &&
+            ((size_t)maxbins * 8 + (size_t)((maxbins + 1) / 2) * 4) * kLanes > (size_t)c->lds_max)
+            wpg = 0;
         if (P.walkers_per_group > 0) wpg = std::min(wpg, (int)P.walkers_per_group);
         if (wpg < 1) return bail(fail(REWL_ERR_INVALID, "window too wide for LDS: " + std::to_string(maxbins) + " bins"));
         if (!tree) {

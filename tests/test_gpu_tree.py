@@ -120,3 +120,11 @@ def test_observables(gpu, model, obs, L, kernel):
                 np.testing.assert_allclose(sums[seen, c] / div, means[seen, c], rtol=1e-9, atol=1e-13,
                                            err_msg=f"walker {g}, column {c}")
             assert np.all(sums[~seen] == 0)
+
+
+def test_moments_keep_the_generic_kernels_window_limit(gpu):
+    """Off the unrolled-row sizes a window with moments is refused above what
+    the generic kernel holds, whatever the number of walkers."""
+    for kernel in ({}, dict(producers=1)):
+        with pytest.raises(abi.REWLError, match="window too wide"):
+            Engine([ising(30, 1, 3, 4.0)], configs.params(observables=1, **kernel))
