@@ -43,8 +43,8 @@ MPIEXEC = "/opt/conda/bin/mpiexec"
 # Measured HBM bytes of one sweep launch of this workload with the default
 # kernel, keyed by sweeps per launch: rocprofv3 --pmc FETCH_SIZE (x 2.0) and
 # WRITE_SIZE (x 1.0), the scales read off a plain 256 MiB copy
-# (profiles/k_sweep_tuned_ising_L64_counters.md).
-MEASURED_TRAFFIC = {1000: (2.0 * 5618.125 + 1.0 * 7537.90625) * 1024}
+# (profiles/k_sweep_tree_ising_L64_counters.md).
+MEASURED_TRAFFIC = {1000: (2.0 * 17504.89 + 1.0 * 8580.0) * 1024}
 
 
 def parse():
@@ -336,10 +336,10 @@ def exact_binned_lng(E_bins, bin_size):
 
 AT_WORKLOADS = {
     "config3": dict(metric="spin-flip attempts/s (Ashkin-Teller L=32)", walkers=512,
-                    data="synthetic (all-up start, Philox draws)", kernel="k_sweep_tuned<AT, L=32>",
+                    data="synthetic (all-up start, Philox draws)", kernel="k_sweep_tree<AT>",
                     workload="2D Ashkin-Teller REWL, L=32, J=1, K=0.5, 1024 bins of width 8, 16 windows x 32 walkers"),
     "config4": dict(metric="spin-flip attempts/s (batched random-strain Ashkin-Teller)", walkers=8192,
-                    data="synthetic (Gaussian strain per realisation, Philox draws)", kernel="k_sweep_field<AT, 3 producers>",
+                    data="synthetic (Gaussian strain per realisation, Philox draws)", kernel="k_sweep_field_tree<AT>",
                     workload="256 random-strain AT realisations, L in {16,24,32,48}, 8 windows x 4 walkers, "
                              "512 bins, one launch per step"),
 }
@@ -347,9 +347,9 @@ AT_WORKLOADS = {
 
 def batched(a):
     """The Ashkin-Teller workloads.  Config 3: one L=32 system, 16 windows x
-    32 walkers, row-unrolled integer kernel.  Config 4: 256 random-strain
+    32 walkers, integer energies.  Config 4: 256 random-strain
     realisations (L in {16, 24, 32, 48}, 8 windows x 4 walkers each, 8192
-    walkers) swept in one launch per step by the field-model kernel.  A step is
+    walkers) swept in one launch per step.  A step is
     sweeps_per_step sweeps + exchange + check.  Attempts/s counts sigma and tau
     proposals (2N per sweep)."""
     from rewl_simulator_amd import configs
@@ -764,25 +764,12 @@ def config2_warm_leg(systems, params, a):
     return out
 
 
-# The walker's instruction stream of the default launch: 24 instructions
-# between successive attempts of the unrolled L = 64 row (the median over the
-# row in the ISA of k_sweep_tuned<0, 64, true, 1, 0>), about 16 of them VALU.
-# A wavefront issues at most one VALU instruction every 4 cycles, so the
-# attempt cannot take fewer than about 4 cycles per instruction.
-WALKER_INSTRUCTIONS_PER_ATTEMPT = 24
-
-
 def latency_model(cycles, clock_ghz, walkers, walkers_per_wave, default_launch):
-    """Cycles per attempt per walker (the walker's chain is the bound of this
-    workload), and for the default launch the issue floor of its instruction
-    stream and the fraction of it reached."""
+    """Cycles per attempt per walker: the walker wavefront's chain is the bound
+    of this workload."""
     out = {"cycles_per_attempt_per_walker": cycles, "clock_ghz_nominal": clock_ghz, "cus": 256}
     if default_launch:
-        floor = 4.0 * WALKER_INSTRUCTIONS_PER_ATTEMPT
-        out.update({"walker_wavefronts": -(-walkers // 33), "walkers_per_wavefront": walkers_per_wave,
-                    "issue_floor": {"instructions_per_attempt": WALKER_INSTRUCTIONS_PER_ATTEMPT,
-                                    "cycles_per_instruction": 4, "floor_cycles": floor,
-                                    "frac": floor / cycles}})
+        out.update({"walker_wavefronts": -(-walkers // walkers_per_wave), "walkers_per_wavefront": walkers_per_wave})
     return out
 
 
@@ -851,12 +838,12 @@ def main():
     att_per_launch = attempts / max(launches, 1)
     achieved = att_per_launch * BYTES_PER_ATTEMPT / avg_launch_s / 1e9
     lnf = min(w["lnf"] for w in (eng.window_info(k) for k in range(eng.num_windows)))
-    default_launch = a.sweep_kernel in (0, 3) and a.producers == 0 and a.walkers_per_group == 0 and not a.observables
+    default_launch = a.sweep_kernel == 0 and a.producers == 0 and a.walkers_per_group == 0 and not a.observables
     traffic = MEASURED_TRAFFIC.get(params["sweeps_per_check"]) if default_launch else None
 
     peak = lds_peak()
     clock_ghz = 2.4
-    walkers_per_wave = W / max(1, -(-W // 33))
+    walkers_per_wave = 4
     cycles = avg_launch_s * clock_ghz * 1e9 / (att_per_launch / W)
     line = {
         "metric": "spin-flip attempts/s; time to ln f=1e-6 (learned warm start vs plain)",
@@ -878,7 +865,7 @@ def main():
             "sweeps_per_step": params["sweeps_per_check"],
             "sweeps_per_exchange": params["sweeps_per_exchange"],
             "attempts_per_step": attempts // a.steps,
-            "parallelism": "one lane per walker, 1 GPU",
+            "parallelism": ("sixteen lanes" if default_launch else "one lane") + " per walker, 1 GPU",
             "producers": a.producers,
             "sweep_kernel": a.sweep_kernel,
             "observables": a.observables,
@@ -894,7 +881,8 @@ def main():
             "frac": achieved / peak,
             "traffic": traffic,
             "peak_source": "rewl_selfcheck(2): 16-byte conflict-free LDS reads on every CU of this GPU",
-            "kernel": "k_sweep_tuned<Ising, L=64> (row-unrolled sweep)" if a.sweep_kernel in (0, 2, 3, 4)
+            "kernel": "k_sweep_tree<Ising> (sixteen lanes per walker)" if default_launch
+                      else "k_sweep_tuned<Ising, L=64> (row-unrolled sweep)" if a.sweep_kernel in (0, 2, 3, 4)
                       else "k_sweep_fast<Ising> (row kernel)",
             "avg_launch_ms": avg_launch_s * 1e3,
             "attempts_per_launch": att_per_launch,

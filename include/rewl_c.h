@@ -166,7 +166,7 @@ typedef struct rewl_params {
                                     rewl_simulation.hpp:401 (unbiased when replicas
                                     also exchange with other windows)               */
     int32_t sweep_kernel;        /* Philox integer path: 0 = auto (sixteen lanes per
-                                    walker in contexts of up to 4096 walkers, else 3
+                                    walker in contexts of few thousand walkers, else 3
                                     for L in {16,24,32,48,64}, else 1); 1 = row
                                     kernel; 2 = row-unrolled; 3 = row-unrolled with
                                     the next slot computed for both outcomes; 4 =
@@ -181,10 +181,10 @@ typedef struct rewl_params {
                                     walker's current bin: |m|, m^2, m^4 (Ising,
                                     ising2d_hamiltonian.hpp:234-256) or the 12 AT
                                     observables (ashkin_teller2d_hamiltonian.hpp:
-                                    267-318); in Philox mode the row-unrolled
-                                    kernel (integer energies, L in {16,24,32,48,64})
-                                    or the field-model kernel keeps them, otherwise
-                                    the generic one.
+                                    267-318); in Philox mode the sixteen-lane and
+                                    row-unrolled kernels (integer energies) or the
+                                    field-model kernel keep them, otherwise the
+                                    generic one.
                                     2: also the Fourier correlators G(qmin) at every
                                     1000th update of a bin (REWL_NUM_OBS_*_CORR
                                     layout).  0: off                                */
