@@ -63,8 +63,9 @@ __device__ __noinline__ double exp_rn_slow(double x) {
 }
 
 // u < RN(exp(x)) for x <= 0 and u = k 2^-32 in [0, 1): the comparison
-// sa_update makes with a correctly rounded exp.  The device exp decides
-// unless u lies within 2^-48 (relative) of it; then the double-double exp.
+// sa_update makes with a correctly rounded exp.  An FP32 exponential decides
+// unless u lies within 1e-5 (relative) of it, then the device exp unless within
+// 2^-48, then the double-double exp.
 __device__ __forceinline__ bool exp_less(double u, double x) {
     if (x == 0.) return u < 1.;
     if (u == 0.) return x > -745.1332191019412;   // RN(exp(x)) > 0

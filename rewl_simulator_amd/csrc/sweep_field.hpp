@@ -1,5 +1,6 @@
 // Wang-Landau sweep, Philox mode, FP64 energies (random-field Ising and
-// random-strain Ashkin-Teller): the throughput kernel for field models.
+// random-strain Ashkin-Teller), one lane per walker: field models whose walkers
+// fill the chip, and their observables (fewer: sweep_field_tree.hpp).
 //
 // Same Markov chain, draws and FP64 arithmetic as k_sweep (and so as the
 // reference's wang_landau_update, wang_landau.hpp:49-93, with the local

@@ -42,7 +42,7 @@
 // (every 1000th update of a bin) is queued by its lane and taken at the end of
 // the row by the whole wavefront, one lattice row per lane.
 //
-// The acceptance bounds come from producer wavefronts (accept_bound.hpp), a
+// The acceptance bounds come from a producer wavefront (accept_bound.hpp), a
 // segment of rows ahead, one barrier per segment.
 //
 // What bounds it: the instruction stream of one wavefront (about 5 cycles an
@@ -50,12 +50,12 @@
 // attempts.  Of the 440 cycles of a step the sixteen instructions of the
 // increments take 85, the FP64 atomic 50 and the count 25; a row adds 320.
 // Measured, cycles per attempt per walker, one lane a walker -> this kernel:
-// L = 64 Ising, 2048 walkers 158 -> 110 (270 -> 187 ms per 1000 sweeps); L = 16,
+// L = 64 Ising, 2048 walkers 158 -> 110 (270 -> 190 ms per 1000 sweeps); L = 16,
 // 8 walkers 253 -> 130; L = 42, 256 walkers (row kernel) 493 -> 112; L = 32
 // Ashkin-Teller, 512 walkers 196 -> 128.  A workgroup has one walker wavefront:
 // two (four) behind one barrier wait for each other and cost 114 at 2048 (137
-// at 4096) where one costs 110 (123); a second producer gained nothing.  Steps of three attempts cost 107 by
-// the same count and two 126.  With observables = 1, one lane a walker -> this
+// at 4096) where one costs 110 (123); a second producer gained nothing.  With the
+// four, steps of three attempts cost 107 by the same count and of two 126.  With observables = 1, one lane a walker -> this
 // kernel: L = 64 Ising 273 -> 157 with 2048 walkers; L = 30 1012 -> 163; L = 32
 // Ashkin-Teller 798 -> 298.  With 2: L = 64 Ising 620 -> 197 (the samples 23 of
 // 172 with 256 walkers), L = 30 2700 -> 191, Ashkin-Teller L = 32

@@ -48,6 +48,12 @@ def test_sizes(gpu, model, L):
              adjust_mode=1 if model == "at" else 0)
 
 
+@pytest.mark.parametrize("L", [16, 24, 32, 48])
+@pytest.mark.parametrize("model", ["ising", "at"])
+def test_one_lane_unrolled_rows(gpu, model, L):
+    run_both([field_system(model, L)], adjust_mode=1 if model == "at" else 0, **ONE_LANE)
+
+
 @pytest.mark.parametrize("kernel", [{}, ONE_LANE])
 @pytest.mark.parametrize("replicas", [1, 2, 5, 64])
 @pytest.mark.parametrize("windows", [1, 3])
