@@ -435,12 +435,15 @@ __device__ __forceinline__ void tree_samples(const KArgs& a, const DevGroup& G, 
         const int j = (int)(what & 15u), block = (int)(what >> 8);
         const int pf = Mdl::flip_plane(__builtin_amdgcn_readlane(fl, 16 * j));
         const uint32_t words = (uint32_t)(o.rec + j * Row::kBytes + Row::kState + 4);
-        uint64_t fw = (uint64_t)((what >> 4) & 15u) << (4 * block);
+        uint32_t fl_lo = 0, fl_hi = 0;   // every block's flips; the row's before `block`
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const uint64_t f = (lds_u32_at(words + (uint32_t)(Row::kWord * i)) >> 4) & 15u;
-            fw |= i < block ? f << (4 * i) : 0ull;
+            const uint32_t f = (lds_u32_at(words + (uint32_t)(Row::kWord * i)) >> 4) & 15u;
+            if (i < 8) fl_lo |= f << (4 * i);
+            else fl_hi |= f << (4 * i - 32);
         }
+        const uint64_t fw = ((((uint64_t)fl_hi << 32) | fl_lo) & ((1ull << (4 * block)) - 1ull)) |
+                            (uint64_t)((what >> 4) & 15u) << (4 * block);
         uint64_t w[NP];
         const uint64_t sites = L == 64 ? ~0ull : (1ull << L) - 1ull;
 #pragma unroll
@@ -458,7 +461,7 @@ __device__ __forceinline__ void tree_samples(const KArgs& a, const DevGroup& G, 
         const double gs = tree_fourier(L, lane, w[0], co, si);
         const double gb = Mdl::kBaxterCorrelator ? tree_fourier(L, lane, w[0] ^ w[NP - 1], co, si) : 0.;
         if (lane == 0) {
-            const int b = (int)((slot - (uint32_t)o.lng) / (uint32_t)T.pitch) - T.guard;
+            const int b = (int)((slot - (uint32_t)o.lng) >> __builtin_ctz((unsigned)T.pitch)) - T.guard;
             double* p = a.obs + (G.hist_base + j + (int64_t)b * kLanes) * a.nobs;
             Mdl::add_correlators([&](int s, double g) { obs_add(p + s, g); }, gs, gb);
         }
