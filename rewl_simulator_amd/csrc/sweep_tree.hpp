@@ -151,6 +151,7 @@ struct TreeLane {
     uint32_t out0, out1;        // outcomes word if its attempt is rejected, accepted: flips << 4, 4 if the last site flipped
     uint32_t l8;                // its walker's column of ln g
     double lnf;
+    int t;                      // its depth: the path's attempts before its own
     int mC, mN;                 // with observables: byte weights of the flips, before and with its attempt
     uint32_t sums;              // with observables: a bin's sums are at ln g's offset x values + this
 };
@@ -358,11 +359,12 @@ __device__ __forceinline__ void tree_block(const TreeLane& c, TreeState& st, Tre
         st.mb = (int)s.w;
         if constexpr (OBS == 2) {
             // counts as they were before the step; the path's earlier updates of
-            // the same bin bring at most three more
+            // the same bin bring at most three more (told by the depth: ln f is 0
+            // while a refinement samples)
             const uint32_t t = acc ? tN : tC;
             if (__builtin_amdgcn_ballot_w64(((t + 3u) & 1023u) < 4u) & path) {
-                const uint32_t before = (c.f1 != 0.0 && sF == s1 ? 1u : 0u) + (c.f2 != 0.0 && sF == s2 ? 1u : 0u) +
-                                        (c.f3 != 0.0 && sF == sC ? 1u : 0u);
+                const uint32_t before = (c.t >= 2 && sF == s1 ? 1u : 0u) + (c.t >= 3 && sF == s2 ? 1u : 0u) +
+                                        (c.t >= 1 && sF == sC ? 1u : 0u);
                 const uint64_t due = __builtin_amdgcn_ballot_w64(((t + before) & 1023u) == 0u) & path;
                 const int lane = threadIdx.x & 63;
                 if ((due >> lane) & 1ull) {
@@ -511,6 +513,7 @@ __device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGrou
                 sel |= 4u << (8 * (i + 1));   // the site after a flip sees its left neighbour flipped
             }
         }
+        c.t = t;
         c.sel0 = sel;
         c.wC = wC;
         c.wN = wC | (T.w << (8 * t));
@@ -537,13 +540,12 @@ __device__ __forceinline__ void sweep_walkers_tree(const KArgs& a, const DevGrou
         c.mN = mC | (1 << (8 * t));
         c.sums = (uint32_t)(o.sums - (o.lng + T.guard * T.pitch) * Mdl::kValues);
     }
-    const int depth = n < 2 ? 0 : n < 4 ? 1 : n < 8 ? 2 : 3;
     const uint32_t latw = (uint32_t)(o.lat + j * (NP * L * o.rowb + 4));
     const uint32_t recw = (uint32_t)(o.rec + j * Row::kBytes);
     // where the lane leaves a step's state: the row's word if it ends the step
-    const uint32_t au = recw + (uint32_t)(depth == 3 ? Row::kState : Row::kSink);
-    const uint32_t au_tail = recw + (uint32_t)(depth == tail - 1 ? Row::kState : Row::kSink);
-    const uint32_t ringw = (uint32_t)(o.ring + j * o.ringw + depth * 8);
+    const uint32_t au = recw + (uint32_t)(c.t == 3 ? Row::kState : Row::kSink);
+    const uint32_t au_tail = recw + (uint32_t)(c.t == tail - 1 ? Row::kState : Row::kSink);
+    const uint32_t ringw = (uint32_t)(o.ring + j * o.ringw + c.t * 8);
     // energy change bytes by the number of disagreeing neighbours; with two
     // couplings biased by 64 each, so that the bytes add without carries, and
     // made signed afterwards

@@ -61,6 +61,41 @@ def test_refine_in_parts_equals_one_call(gpu):
     one.close(); parts.close()
 
 
+@pytest.mark.parametrize("cadence", [1, 5, 50])
+@pytest.mark.parametrize("obs", [1, 2])
+@pytest.mark.parametrize("model", ["ising", "at"])
+def test_refine_with_observables_matches_oracle(gpu, model, obs, cadence):
+    """Sampling with ln f = 0 while observables are kept, every bin past
+    several multiples of 1000 updates (the correlator's samples): chains and
+    histograms bit for bit, the refined ln g, sums and samples."""
+    print(f"case: refine with observables={obs} model={model} cadence={cadence}", flush=True)
+    s = configs.ising_full_range(8, 4.0, 3, 3) if model == "ising" else configs.at_system(6, -180.0, 4.0, 8.0, 3, 3)
+    p = configs.params(flatness_mode=abi.FLAT_MIN_OVER_MEAN, flatness=0.5, schedule=abi.SCHED_HALVE, observables=obs,
+                       lnf_final=1e-2, sweeps_per_check=50, sweeps_per_exchange=50, adjust_mode=1)
+    eng, ora = Engine([s], p), Oracle([s], p)
+    eng.adjust_to_range(); ora.adjust_to_range()
+    eng.run(40); ora.run(40)
+    eng.refine(3000, cadence); ora.refine(3000, cadence)
+    corr = eng.correlator_slots(s["model"])
+    boundaries = 0
+    for g in range(eng.num_walkers):
+        assert eng.energy(g) == ora.state(g)["E"], g
+        np.testing.assert_array_equal(eng.spins(g), ora.spins(g))
+        np.testing.assert_array_equal(eng.visits(g), ora.visits(g), err_msg=f"histogram of walker {g}")
+        np.testing.assert_allclose(eng.logdos(g), ora.logdos(g), rtol=4e-16, atol=4e-15)
+        sums = eng.observables(g)
+        means, n = ora.observables(g)   # n: every update, those before the refinement too
+        seen = n > 0
+        boundaries += int((n // 1000).sum())
+        for c in range(sums.shape[1]):
+            div = np.ceil(n[seen] / 1000.0) if c in corr else n[seen]
+            np.testing.assert_allclose(sums[seen, c] / div, means[seen, c], rtol=1e-9, atol=1e-13,
+                                       err_msg=f"walker {g}, column {c}")
+        assert np.all(sums[~seen] == 0)
+    assert boundaries > 100 * eng.num_walkers
+    eng.close(); ora.close()
+
+
 def test_refined_lng_within_0_01_of_exact_L16(gpu):
     """2D Ising L = 16 (the first workload's lattice: full spectrum, bins of
     4, 4 windows at 75% overlap), here 128 walkers per window: Wang-Landau to
