@@ -14,7 +14,9 @@
 #include <cstdio>
 #include <cstring>
 #include <limits>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <numeric>
 #include <random>
 #include <string>
@@ -22,6 +24,7 @@
 
 #include "../../include/rewl_c.h"
 #include "aux_kernels.hpp"
+#include "replay_fill.hpp"
 #include "sweep.hpp"
 #include "sweep_fast.hpp"
 #include "sweep_field.hpp"
@@ -400,26 +403,27 @@ int replay_topup(rewl_ctx* c, uint64_t need) {
     HIP_TRY(hipMemcpyAsync(cur.data(), c->d_w_cursor.p, (size_t)W * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     const uint64_t C = c->ring_cap;
-    uint64_t words = 0;
-    for (int g = 0; g < W; ++g) words += cur[g] + C - std::min(cur[g] + C, c->filled[g]);
-    std::vector<uint64_t> tmp(words);
-    uint64_t* t = tmp.data();
-    for (int g = 0; g < W; ++g) {
-        const uint64_t target = cur[g] + C;
-        uint64_t& f = c->filled[g];
-        while (f < target) {
-            const uint64_t pos = f & (C - 1);
-            const uint64_t len = std::min<uint64_t>(target - f, C - pos);
-            for (uint64_t k = 0; k < len; ++k) t[k] = c->engines[g]();
-            HIP_TRY(hipMemcpyAsync(c->d_ring.p + (size_t)g * C + pos, t, len * sizeof(uint64_t), hipMemcpyHostToDevice,
-                                   c->stream));
-            t += len;
-            f += len;
-        }
-    }
-    HIP_TRY(hipMemcpyAsync(c->d_ring_filled.p, c->filled.data(), (size_t)W * sizeof(uint64_t), hipMemcpyHostToDevice,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));   // tmp goes
+    const uint64_t room = std::min(replay_lack(W, cur.data(), c->filled.data(), C), kReplayStage);
+    const std::unique_ptr<uint64_t[]> stage(new (std::nothrow) uint64_t[room]);
+    if (!stage) return fail(REWL_ERR_DEVICE, "no host memory for the replay streams");
+    hipError_t e = hipSuccess;
+    const bool filled = replay_fill(
+        W, cur.data(), c->filled.data(), C, stage.get(), room, [&](int g) { return c->engines[g](); },
+        [&](int g, uint64_t pos, const uint64_t* w, uint64_t n) {
+            e = hipMemcpyAsync(c->d_ring.p + (size_t)g * C + pos, w, n * sizeof(uint64_t), hipMemcpyHostToDevice,
+                               c->stream);
+            return e == hipSuccess;
+        },
+        [&] {
+            e = hipStreamSynchronize(c->stream);
+            return e == hipSuccess;
+        });
+    if (filled)
+        e = hipMemcpyAsync(c->d_ring_filled.p, c->filled.data(), (size_t)W * sizeof(uint64_t), hipMemcpyHostToDevice,
+                           c->stream);
+    const hipError_t waited = hipStreamSynchronize(c->stream);   // stage goes
+    HIP_TRY(e);
+    HIP_TRY(waited);
     c->replay_left = C - std::min(need, C);
     return REWL_OK;
 }
