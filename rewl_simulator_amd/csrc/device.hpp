@@ -8,7 +8,9 @@
 //     lat[group.lat_base + (plane * L + y) * 64 + j]; bit x of the word is the
 //     spin at site y*L + x, bit = 1 meaning spin -1 (so all-up is all zeros);
 //   * histogram bin b of that walker lives at [group.hist_base + b * 64 + j] in
-//     lng (FP64), cnt (u32) and visits (u64).
+//     lng (FP64), cnt (u32) and visits (u64);
+//   * the groups of the sixteen-lanes-a-walker kernels have four walkers, and
+//     sixteen groups lie side by side in a row of 64 (place_tree_groups).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

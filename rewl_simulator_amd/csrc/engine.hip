@@ -696,6 +696,60 @@ int max_ndof(const rewl_ctx* c) {
     return m;
 }
 
+// A launch has one workgroup per group and the dispatcher starts them in
+// list order: the longest first (attempts per sweep, DoF of the system),
+// so that when a batch has more groups than the chip holds, the groups
+// that start last are short ones (longest-processing-time order).
+void longest_first(const rewl_ctx* c, std::vector<int32_t>& list) {
+    std::stable_sort(list.begin(), list.end(), [&](int32_t x, int32_t y) {
+        return c->sys[(size_t)c->groups[(size_t)x].sys].ndof > c->sys[(size_t)c->groups[(size_t)y].sys].ndof;
+    });
+}
+
+// The rows of the four-walker groups' lattices and histograms.  A row is kLanes
+// wide and sixteen consecutive groups share it: with rows of their own they
+// took sixteen times the memory, which creation and the passes over all
+// walkers went through (512 Ashkin-Teller walkers with observables 2 created in
+// 1.38 ms instead of 0.91; 256 replicas in 16 windows at L = 64 finalized in
+// 669 us instead of 555).  Workgroups go to the eight XCDs in turn, and a line that
+// two XCDs write costs (a sweep and exchange of 2048 walkers at L = 64 1.2 %
+// when neighbours on the list shared rows), so the list takes groups of eight
+// rows in turn: the sixteen of a row run on one XCD.  Fewer than 128 groups
+// of a size are spread over eight rows likewise.
+void place_tree_groups(rewl_ctx* c) {
+    constexpr size_t kXcds = 8, kSides = kLanes / kTreePerWave;
+    for (auto& list : c->tree_groups) {
+        longest_first(c, list);
+        auto ndof = [&](size_t i) { return c->sys[(size_t)c->groups[(size_t)list[i]].sys].ndof; };
+        std::vector<int32_t> order(list.size());
+        for (size_t first = 0, n; first < list.size(); first += n) {
+            for (n = 1; n < kXcds * kSides && first + n < list.size() && ndof(first + n) == ndof(first);) ++n;
+            size_t next = first;   // groups of rows 0, 1, ... one after the other
+            for (size_t x = 0; x < std::min(kXcds, n); ++x) {
+                const size_t sides = n / kXcds + (x < n % kXcds ? 1 : 0);
+                size_t nb = 0;
+                for (size_t side = 0; side < sides; ++side) {
+                    const int32_t gid = list[next + side];
+                    DevGroup& G = c->groups[(size_t)gid];
+                    G.hist_base = (int64_t)(c->hist_total + side * kTreePerWave);
+                    G.lat_base = (int64_t)(c->lat_total + side * kTreePerWave);
+                    for (int j = 0; j < G.nwalkers; ++j) {
+                        c->w_hist[(size_t)(G.first_walker + j)] = G.hist_base + j;
+                        c->w_lat[(size_t)(G.first_walker + j)] = G.lat_base + j;
+                    }
+                    nb = std::max(nb, (size_t)G.nbins);
+                    order[first + x + side * kXcds] = gid;
+                }
+                const HostSystem& S = c->sys[(size_t)c->groups[(size_t)list[next]].sys];
+                c->hist_total += nb * kLanes;
+                c->lat_total += (size_t)model_info(S.d.model).planes * (size_t)S.d.L * kLanes;
+                next += sides;
+            }
+        }
+        list.swap(order);
+    }
+}
+
 // Device buffers of one rewl_anneal call, released on every return path.
 struct AnnealBuffers {
     DevBuf<DevSystem> sys;
@@ -939,10 +993,12 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
             int nb = 0;
             for (int j = 0; j < G.nwalkers; ++j) nb = std::max(nb, c->win[c->w_window[G.first_walker + j]].nbins);
             G.nbins = nb;
-            G.hist_base = (int64_t)c->hist_total;
-            G.lat_base = (int64_t)c->lat_total;
-            c->hist_total += (size_t)nb * kLanes;
-            c->lat_total += (size_t)planes * S.d.L * kLanes;
+            if (!tree) {   // else place_tree_groups
+                G.hist_base = (int64_t)c->hist_total;
+                G.lat_base = (int64_t)c->lat_total;
+                c->hist_total += (size_t)nb * kLanes;
+                c->lat_total += (size_t)planes * S.d.L * kLanes;
+            }
             const int gid = (int)c->groups.size();
             for (int j = 0; j < G.nwalkers; ++j) {
                 const int g = G.first_walker + j;
@@ -1001,6 +1057,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         else if (packed <= (size_t)c->lds_max) c->class_packed[cls] = true;
         else return bail(fail(REWL_ERR_INVALID, "window too wide for LDS: " + std::to_string(nb) + " bins"));
     }
+    place_tree_groups(c);
     c->flush_every = std::max(1, 65535 / (max_ndof(c) + 1));
 
     // ---- exchange pair lists ---------------------------------------------------
@@ -1056,18 +1113,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
     if ((rc = upload(c->d_w_local, c->w_local, c->stream))) return bail(rc);
     if ((rc = upload(c->d_w_hist, c->w_hist, c->stream))) return bail(rc);
     if ((rc = upload(c->d_w_lat, c->w_lat, c->stream))) return bail(rc);
-    // A launch has one workgroup per group and the dispatcher starts them in
-    // list order: the longest first (attempts per sweep, DoF of the system),
-    // so that when a batch has more groups than the chip holds, the groups
-    // that start last are short ones (longest-processing-time order).
-    for (int cls = 0; cls < 4; ++cls)
-        std::stable_sort(c->class_groups[cls].begin(), c->class_groups[cls].end(), [&](int32_t x, int32_t y) {
-            return c->sys[(size_t)c->groups[(size_t)x].sys].ndof > c->sys[(size_t)c->groups[(size_t)y].sys].ndof;
-        });
-    for (auto& list : c->tree_groups)
-        std::stable_sort(list.begin(), list.end(), [&](int32_t x, int32_t y) {
-            return c->sys[(size_t)c->groups[(size_t)x].sys].ndof > c->sys[(size_t)c->groups[(size_t)y].sys].ndof;
-        });
+    for (int cls = 0; cls < 4; ++cls) longest_first(c, c->class_groups[cls]);
     for (int m = 0; m < 4; ++m)
         if ((rc = upload(c->d_tree_groups[m], c->tree_groups[m], c->stream))) return bail(rc);
     if ((rc = upload(c->d_tree_scale, tree_scales, c->stream))) return bail(rc);

@@ -2,6 +2,8 @@
 oracle, bit for bit: lattice sizes around its blocks of four sites and its
 dword of four blocks, groups whose last wavefront is partly empty, windows of
 different widths, couplings and bin sizes at the ends of its byte scales."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -128,3 +130,32 @@ def test_moments_keep_the_generic_kernels_window_limit(gpu):
     for kernel in ({}, dict(producers=1)):
         with pytest.raises(abi.REWLError, match="window too wide"):
             Engine([ising(30, 1, 3, 4.0)], configs.params(observables=1, **kernel))
+
+
+def free_memory():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL("libamdhip64.so").hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("model,field", [("ising", False), ("at", False), ("ising", True)])
+def test_memory_of_a_context(gpu, model, field):
+    """Groups of four walkers share rows: a context holds little more than its
+    walkers' histograms (8 + 4 + 8 bytes per bin, and the observables), not a
+    row of 64 lanes for each group."""
+    s = ising(32, 2, 256, 2.0) if model == "ising" else ashkin_teller(32, 4, 256, 16.0)
+    obs = 0 if field or model == "ising" else 2
+    if field:
+        h = configs.gaussian_strain(32, 0.5, 3)
+        lo = -2.0 * 1024 - float(np.abs(h).sum())
+        s = configs.ising_system(32, lo, lo + 900 * 3.0, 3.0, 2, 256, field=h)
+    with Engine([s], configs.params(observables=obs)):   # whatever the first context sets up
+        pass
+    before = free_memory()
+    with Engine([s], configs.params(observables=obs)) as eng:
+        held = before - free_memory()
+        bins = sum(s["replicas_per_window"] * w["num_bins"] for w in eng.windows)
+    per = 20 + (16 * 8 + 4 if obs else 0)
+    # rows are as long as their widest window; the same again is left for it
+    # and for the granularity of allocations
+    assert held <= 2 * per * bins + (16 << 20)
