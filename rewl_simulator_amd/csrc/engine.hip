@@ -25,6 +25,7 @@
 #include "../../include/rewl_c.h"
 #include "aux_kernels.hpp"
 #include "replay_fill.hpp"
+#include "sweep_choice.hpp"
 #include "sweep.hpp"
 #include "sweep_fast.hpp"
 #include "sweep_field.hpp"
@@ -119,18 +120,6 @@ std::vector<HostWindow> make_windows(const rewl_system_desc& d) {
 
 bool integral(double v) { return std::isfinite(v) && std::floor(v) == v && std::fabs(v) < 1e9; }
 
-// k_sweep_tree takes contexts of at most this many walkers: 1280 workgroups of
-// four walkers, five per CU; beyond, its time per attempt grows with the walkers
-// while the kernels with one lane per walker still have room.  Measured, cycles
-// per attempt, tree against lane: L = 64 Ising 103 / 161 at 512 walkers, 110 /
-// 159 at 2048, 131 / 164 at 4096, 161 / 165 at 5120, 246 / 168 at 6144; L = 32
-// Ashkin-Teller 129 / 198, 141 / 198 at 4096, 184 / 198, 236 / 198.  Sizes
-// without an unrolled-row kernel have the row kernel to compare with (470-530
-// cycles): 225 at 8192.  With observables the sums take the LDS of the walkers
-// that would share a CU: with moments L = 64 Ising 348 / 564 at 4096, L = 16
-// Ashkin-Teller 641 / 845 at 4096 and 858 / 845 at 5120, L = 20 636 / 1513 and
-// 1338 / 1520.
-constexpr int kTreeMaxWalkers = 5120, kTreeMaxWalkersRow = 12288, kTreeMaxWalkersObs = 4096;
 // k_sweep_field_tree takes the FP64 systems of a context as long as their
 // walkers, each counted as its system's degrees of freedom over the largest
 // system's, are at most this many: 1024 workgroups, four per CU (registers and
@@ -487,6 +476,26 @@ int launch_sweep_field(rewl_ctx* c, int cls, int nsweeps) {
 // (sweep_tuned.hpp); otherwise none.
 size_t tuned_obs_bytes(int model, int observables) {
     return observables >= 1 ? 8 * (size_t)model_info(model).values : 0;
+}
+
+// A system in the row-unrolled kernel: guard bins (|Delta E| <= 4 (2J) (+ 4
+// (2K)) on the integer path), LDS of a walker, walkers of a workgroup.
+struct TunedShape {
+    int guard, walkers;
+    size_t per_walker;
+};
+TunedShape tuned_shape(const rewl_ctx* c, const HostSystem& S, int maxbins) {
+    TunedShape t;
+    const long long maxde =
+        4LL * std::abs(S.twoJ) + (model_info(S.d.model).product_coupling ? 4LL * std::abs(S.twoK) : 0LL);
+    const long long bs = (long long)c->win[S.first_window].bs;
+    t.guard = (int)((maxde + bs - 1) / bs) + 1;
+    t.per_walker = (size_t)(maxbins + 2 * t.guard) * kTunedSlot + (size_t)tuned_ring_stride(S.d.L) +
+                   (size_t)maxbins * tuned_obs_bytes(S.d.model, c->p.observables);
+    // observables = 2: the cos/sin table of the correlator after the rings
+    const size_t room = (size_t)c->lds_max - (c->p.observables == 2 ? 16 * (size_t)S.d.L : 0);
+    t.walkers = std::min(kLanes, (int)(room / t.per_walker));
+    return t;
 }
 
 // Philox mode, integer path, L in kTunedL: the row-unrolled kernel (sweep_tuned.hpp).
@@ -864,28 +873,60 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
 
     // ---- systems swept with sixteen lanes a walker -------------------------------
     // When the caller asks for no particular kernel or launch shape and the
-    // context has few enough walkers (kTreeMaxWalkers, kFieldTreeMaxWalkers).
+    // context has few enough walkers (sweep_choice.hpp, kFieldTreeMaxWalkers).
     std::vector<uint8_t> tree_sys(c->sys.size(), 0);
     std::vector<TreeScale> tree_scales(c->sys.size());
     {
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
         const bool shape_free = P.rng_mode == REWL_RNG_PHILOX && P.sweep_kernel == 0 && P.producers == 0 &&
                                 P.walkers_per_group == 0 && !P.densities;
-        auto fits = [&](const HostSystem& S, TreeScale* t) {
-            if (!tree_scale(S.d, S.twoJ, S.twoK, t)) return false;
+        auto max_bins = [&](const HostSystem& S) {
             int nb = 1;
             for (int k = 0; k < S.d.num_windows; ++k) nb = std::max(nb, c->win[S.first_window + k].nbins);
-            const long long bytes = (long long)(nb + 2 * t->guard) * t->pitch * 2;
-            if (bytes > 4LL * c->lds_max) return false;   // keeps the sums below in range
-            const ModelInfo m = model_info(S.d.model);
-            return (size_t)tree_lds(m.planes, S.d.L, nb, t->pitch, t->guard, P.observables, m.values).total <=
-                   (size_t)c->lds_max;
+            return nb;
         };
+        // bytes of LDS of a workgroup, 0 if the kernel does not take the system
+        auto group_lds = [&](const HostSystem& S, TreeScale* t) -> size_t {
+            if (!tree_scale(S.d, S.twoJ, S.twoK, t)) return 0;
+            const int nb = max_bins(S);
+            const long long bytes = (long long)(nb + 2 * t->guard) * t->pitch * 2;
+            if (bytes > 4LL * c->lds_max) return 0;   // keeps the sums below in range
+            const ModelInfo m = model_info(S.d.model);
+            const size_t lds = (size_t)tree_lds(m.planes, S.d.L, nb, t->pitch, t->guard, P.observables, m.values).total;
+            return lds <= (size_t)c->lds_max ? lds : 0;
+        };
+        // Of a model's systems with an unrolled row: workgroups and largest LDS
+        // here and, by lattice side, with one lane per walker.
+        struct Launch {
+            long long groups = 0, lds = 0;
+        } tree_launch[2], lane_launch[2][5];
         for (size_t si = 0; shape_free && si < c->sys.size(); ++si) {
             const HostSystem& S = c->sys[si];
-            if (W > (P.observables ? kTreeMaxWalkersObs : tuned_index(S.d.L) >= 0 ? kTreeMaxWalkers : kTreeMaxWalkersRow))
-                continue;
+            const int li = tuned_index(S.d.L), walkers = S.d.num_windows * S.d.replicas_per_window;
+            if (W > tree_walker_limit(model_info(S.d.model).planes, S.d.L, P.observables, li >= 0)) continue;
             if (!S.intpath || S.d.L < kTreeMinL || !simple_range(S, c->win)) continue;
-            if (fits(S, &tree_scales[si])) tree_sys[si] = 1;
+            const size_t lds = group_lds(S, &tree_scales[si]);
+            tree_sys[si] = lds > 0;
+            if (!lds || li < 0) continue;
+            const TunedShape t = tuned_shape(c, S, max_bins(S));
+            if (t.walkers < 1) continue;
+            auto add = [&](Launch& l, int per, size_t bytes) {
+                l.groups += (walkers + per - 1) / per;
+                l.lds = std::max(l.lds, (long long)bytes);
+            };
+            add(tree_launch[S.d.model], kTreePerWave, lds);
+            add(lane_launch[S.d.model][li], t.walkers, (size_t)t.walkers * t.per_walker);
+        }
+        for (int m = 0; m < 2; ++m) {
+            long long lane_rounds = 0;
+            for (const Launch& l : lane_launch[m]) lane_rounds += workgroup_rounds(l.groups, l.lds, c->lds_max, cus);
+            const Launch& l = tree_launch[m];
+            if (tree_pays(P.observables, workgroup_rounds(l.groups, l.lds, c->lds_max, cus),
+                          workgroups_per_cu(l.lds, c->lds_max) == 1, lane_rounds))
+                continue;
+            for (size_t si = 0; si < c->sys.size(); ++si)
+                if (c->sys[si].d.model == m && tuned_index(c->sys[si].d.L) >= 0) tree_sys[si] = 0;
         }
         int64_t attempts = 0, largest = 1;   // of the FP64 systems, per sweep: all walkers', one walker's at most
         for (const HostSystem& S : c->sys) {
@@ -897,8 +938,7 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
         for (size_t si = 0; shape_free && !P.observables && few && si < c->sys.size(); ++si) {
             const HostSystem& S = c->sys[si];
             if (S.intpath || S.d.L < kTreeMinL) continue;
-            int nb = 1;
-            for (int k = 0; k < S.d.num_windows; ++k) nb = std::max(nb, c->win[S.first_window + k].nbins);
+            const int nb = max_bins(S);
             if ((long long)nb * 12 * kTreePerWave > c->lds_max) continue;   // keeps the sum below in range
             const ModelInfo m = model_info(S.d.model);
             if (field_tree_lds(m.planes, m.energy_terms, S.d.L, nb).total <= c->lds_max) tree_sys[si] = 1;
@@ -939,18 +979,11 @@ int rewl_create(const rewl_system_desc* systems, int32_t num_systems, const rewl
                                                "and no densities"));
         const bool field_tree = tree && !S.intpath;
         int wpg = tree ? kTreePerWave : kLanes;
-        // guard bins: |Delta E| <= 4 (2J) (+ 4 (2K)) on the integer path
         int guard = 0;
         if (tuned) {
-            const long long maxde =
-                4LL * std::abs(S.twoJ) + (model_info(S.d.model).product_coupling ? 4LL * std::abs(S.twoK) : 0LL);
-            const long long bs = (long long)c->win[S.first_window].bs;
-            guard = (int)((maxde + bs - 1) / bs) + 1;
-            // observables = 2: the cos/sin table of the correlator after the rings
-            const size_t room = (size_t)c->lds_max - (P.observables == 2 ? 16 * (size_t)S.d.L : 0);
-            wpg = std::min(kLanes, (int)(room / ((size_t)(maxbins + 2 * guard) * kTunedSlot +
-                                                 (size_t)tuned_ring_stride(S.d.L) +
-                                                 (size_t)maxbins * tuned_obs_bytes(S.d.model, P.observables))));
+            const TunedShape t = tuned_shape(c, S, maxbins);
+            guard = t.guard;
+            wpg = t.walkers;
         }
         else if (fast && !tree)
             wpg = std::min(kLanes, (int)((size_t)c->lds_max /

@@ -94,3 +94,24 @@ def test_mixed_context(gpu):
     clean = configs.ising_system(9, -2 * N, -2 * N + 4.0 * np.ceil(N / 2), 4.0, 2, 3, seed=3)
     run_both([field_system("ising", 13, 2, 2, seed=7), clean, field_system("at", 16, 3, 2, seed=9),
               field_system("at", 7, 2, 5, seed=11)], sweeps=7, adjust_mode=1)
+
+
+@pytest.mark.parametrize("model", ["ising", "at"])
+@pytest.mark.parametrize("more", [0, 1])
+def test_on_either_side_of_the_choice(gpu, model, more):
+    """4096 walkers of one size, the most that the sixteen-lane sweep takes, and
+    a few more: the chain is the same."""
+    s = [field_system(model, 9, 4, r, seed=k + 1) for k, r in enumerate([256] * 4 + [1] * more)]
+    p = configs.params(lnf_initial=0.05, adjust_mode=1)
+    with Engine(s, p) as eng:
+        ora = Oracle(s, p)
+        eng.adjust_to_range(); ora.adjust_to_range()
+        for _ in range(2):
+            eng.sweeps(2); ora.sweeps(2)
+            eng.exchange(); ora.exchange()
+        window_states_equal(eng, ora)
+        for g in range(0, eng.num_walkers, 23):
+            assert eng.energy(g) == ora.state(g)["E"], g
+            np.testing.assert_array_equal(eng.spins(g), ora.spins(g))
+            np.testing.assert_array_equal(eng.logdos(g).view(np.uint64), ora.logdos(g).view(np.uint64))
+            np.testing.assert_array_equal(eng.counts(g).astype(np.uint64), ora.counts(g))

@@ -159,3 +159,28 @@ def test_memory_of_a_context(gpu, model, field):
     # rows are as long as their widest window; the same again is left for it
     # and for the granularity of allocations
     assert held <= 2 * per * bins + (16 << 20)
+
+
+@pytest.mark.parametrize("model,L,obs,copies,replicas", [
+    ("ising", 5, 0, 2, (192, 193)), ("at", 6, 0, 2, (192, 193)), ("ising", 9, 0, 3, (213, 214)), ("at", 16, 0, 2, (160, 161)),
+    ("ising", 32, 0, 2, (128, 129)), ("ising", 9, 1, 2, (128, 129)), ("at", 16, 2, 2, (128, 129)),
+    ("ising", 64, 1, 1, (192, 193)), ("at", 64, 0, 1, (192, 193))])
+def test_on_either_side_of_the_choice(gpu, model, L, obs, copies, replicas):
+    """Contexts at and just past what the sixteen-lane sweep takes, by walkers
+    or (L = 64) by windows so wide that LDS decides: the chain is the same."""
+    for R in replicas:
+        s = ising(L, 16, R, 8.0 if L == 64 else 4.0) if model == "ising" else ashkin_teller(L, 16, R)
+        systems = [dict(s, seed=77 + k) for k in range(copies)]
+        p = configs.params(lnf_initial=0.05, observables=obs, adjust_mode=1)
+        with Engine(systems, p) as eng:
+            ora = Oracle(systems, p)
+            eng.adjust_to_range(); ora.adjust_to_range()
+            for _ in range(2):
+                eng.sweeps(1); ora.sweeps(1)
+                eng.exchange(); ora.exchange()
+            window_states_equal(eng, ora)
+            for g in range(0, eng.num_walkers, 23):
+                assert eng.energy(g) == ora.state(g)["E"], g
+                np.testing.assert_array_equal(eng.spins(g), ora.spins(g))
+                np.testing.assert_array_equal(eng.logdos(g).view(np.uint64), ora.logdos(g).view(np.uint64))
+                np.testing.assert_array_equal(eng.counts(g).astype(np.uint64), ora.counts(g))
