@@ -1,14 +1,17 @@
 """Launch-shape autotuner for the sweep kernels.
 
 For a workload (list of systems + params) it times short sweeps of a scratch
-context for each candidate launch shape and returns the fastest:
+context for each candidate launch shape and returns the fastest.  The first
+candidate is always the automatic shape, everything 0, which the engine chooses
+by the workload (sixteen lanes a walker where walkers are few); the others are
 
   * integer energies, Philox draws: the row-unrolled kernel's variants
-    (sweep_kernel 0 = slot speculation, 2 = none, 4 = read-ahead) with 7 or 3
+    (sweep_kernel 3 = slot speculation, 2 = none, 4 = read-ahead) with 7 or 3
     producer wavefronts, and the row kernel (sweep_kernel 1);
-  * field models, Philox draws: the field kernel (producers 0) or the generic
-    kernel (producers -1), with the LDS-fitting group width or 16 walkers;
-  * replay mode: the generic kernel at the LDS-fitting group width or 32.
+  * field models, Philox draws: the field kernel with one lane per walker
+    (producers 1) or the generic kernel (producers -1), with the LDS-fitting
+    group width or 16 walkers;
+  * replay mode: the generic kernel with 32 walkers a group.
 
 Results are cached per workload signature (in memory, and in a JSON file when
 a path is given).  The choice changes only speed: every launch shape runs
@@ -25,13 +28,19 @@ from .engine import Engine
 _CACHE = {}
 
 
+# Goes into the signature: raised when the candidates or what a shape runs
+# change, so that a cache file does not pin choices made among other kernels.
+VERSION = 2
+
+
 def signature(systems, params):
     items = []
     for s in systems:
         items.append((s["model"], s["L"], s["J"], s["K"], s["field"] is not None if "field" in s else False,
                       s["num_windows"], s["replicas_per_window"], round(s["e_max"] - s["e_min"], 6), s["bin_size"]))
     items.sort()
-    h = hashlib.sha1(json.dumps([items, params.get("rng_mode", 0)], default=str).encode()).hexdigest()[:16]
+    h = hashlib.sha1(json.dumps([VERSION, items] + [params.get(k, 0) for k in ("rng_mode", "observables", "densities")],
+                                default=str).encode()).hexdigest()[:16]
     return h
 
 
@@ -41,17 +50,15 @@ TUNED_L = (16, 24, 32, 48, 64)
 def candidates(systems, params):
     intpath = all(s.get("field") is None and s.get("h", 0.0) == 0.0 for s in systems)
     philox = params.get("rng_mode", abi.RNG_PHILOX) == abi.RNG_PHILOX
+    auto = dict(walkers_per_group=0, producers=0, sweep_kernel=0)
+    out = [auto]
     if not philox:
-        return [dict(walkers_per_group=w, producers=0, sweep_kernel=0) for w in (0, 32)]
+        return out + [dict(auto, walkers_per_group=32)]
     if not intpath:
-        return [dict(walkers_per_group=w, producers=p, sweep_kernel=0) for p in (0, -1) for w in (0, 16)]
-    out = []
+        return out + [dict(auto, walkers_per_group=w, producers=p) for p in (1, -1) for w in (0, 16)]
     if all(s["L"] in TUNED_L for s in systems):
-        for sk in (0, 2, 4):
-            for prod in (0, 3):
-                out.append(dict(walkers_per_group=0, producers=prod, sweep_kernel=sk))
-    out.append(dict(walkers_per_group=0, producers=0, sweep_kernel=1))
-    return out
+        out += [dict(auto, sweep_kernel=sk, producers=prod) for sk in (3, 2, 4) for prod in (0, 3)]
+    return out + [dict(auto, sweep_kernel=1)]
 
 
 def measure(systems, params, shape, sweeps):
