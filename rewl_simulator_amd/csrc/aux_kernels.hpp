@@ -169,6 +169,10 @@ __device__ __forceinline__ void wave_shuffle(int* v, int* pos, int n, int first,
             pos[1] = (int)k;
         }
     }
+    // the lanes read one another's positions: the compiler keeps the order of the
+    // LDS operations, which end in order within a wavefront
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     if (__builtin_amdgcn_ballot_w64(in_order)) {
         if (lane == 0) shuffle_partners(v, n, st);
         return;
