@@ -150,6 +150,7 @@ __device__ void shuffle_partners(int* v, int n, ExchStream& st) {
 // (or lie beyond a replay stream) sends lane 0 through them in order.  v, pos:
 // LDS, n ints each; the cursor is lane 0's.
 __device__ __forceinline__ void wave_shuffle(int* v, int* pos, int n, int first, ExchStream& st, int lane) {
+    if (n < 2) return;   // no draw
     const int odd = n & 1, draws = n / 2;   // n even: the first draw makes one swap
     bool in_order = false;
     for (int d = lane; d < draws; d += kLanes) {
