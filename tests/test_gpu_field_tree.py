@@ -115,3 +115,16 @@ def test_on_either_side_of_the_choice(gpu, model, more):
             np.testing.assert_array_equal(eng.spins(g), ora.spins(g))
             np.testing.assert_array_equal(eng.logdos(g).view(np.uint64), ora.logdos(g).view(np.uint64))
             np.testing.assert_array_equal(eng.counts(g).astype(np.uint64), ora.counts(g))
+
+
+@pytest.mark.parametrize("kernel", [{}, ONE_LANE])
+@pytest.mark.parametrize("model", ["ising", "at"])
+@pytest.mark.parametrize("L", [24, 32, 48])
+def test_energies_on_bin_edges_of_unrolled_rows(gpu, model, L, kernel):
+    """The same on the sides whose rows the kernel with one lane a walker
+    unrolls: a field of multiples of 1/2 and bins of 3."""
+    h = np.round(2.0 * configs.gaussian_strain(L, 1.0, 200 + L)) / 2.0
+    N, span = L * L, float(np.ceil(np.abs(h).sum())) + 8.0
+    s = (configs.ising_system(L, -2.0 * N - span, 2.0 * N + span, 3.0, 6, 2, field=h) if model == "ising" else
+         configs.at_system(L, -5.0 * N - span, 3.0 * N + span, 3.0, 6, 2, field=h))
+    run_both([s], adjust_mode=1 if model == "at" else 0, **kernel)
