@@ -336,13 +336,31 @@ def exact_binned_lng(E_bins, bin_size):
 
 AT_WORKLOADS = {
     "config3": dict(metric="spin-flip attempts/s (Ashkin-Teller L=32)", walkers=512,
-                    data="synthetic (all-up start, Philox draws)", kernel="k_sweep_tree<AT>",
+                    data="synthetic (all-up start, Philox draws)",
                     workload="2D Ashkin-Teller REWL, L=32, J=1, K=0.5, 1024 bins of width 8, 16 windows x 32 walkers"),
     "config4": dict(metric="spin-flip attempts/s (batched random-strain Ashkin-Teller)", walkers=8192,
-                    data="synthetic (Gaussian strain per realisation, Philox draws)", kernel="k_sweep_field_tree<AT>",
+                    data="synthetic (Gaussian strain per realisation, Philox draws)",
                     workload="256 random-strain AT realisations, L in {16,24,32,48}, 8 windows x 4 walkers, "
                              "512 bins, one launch per step"),
 }
+
+
+def sweep_kernel_of(a):
+    """(kernel, lanes per walker) that the engine runs on a workload with the
+    launch shape and observables asked for (rewl_create's choice; these
+    workloads' walkers and windows are within what sixteen lanes take)."""
+    auto = a.sweep_kernel == 0 and a.producers == 0 and a.walkers_per_group == 0
+    model = "Ising" if a.workload == "config2" else "AT"
+    row_kernels = a.producers >= 0 and a.sweep_kernel != 1
+    if a.workload == "config4":   # FP64 energies
+        if auto and not a.observables:
+            return f"k_sweep_field_tree<{model}>", 16
+        return (f"k_sweep_field<{model}>" if row_kernels and a.observables < 2 else f"k_sweep<{model}>"), 1
+    if auto:
+        return f"k_sweep_tree<{model}>", 16
+    if row_kernels:
+        return f"k_sweep_tuned<{model}> (row-unrolled)", 1
+    return (f"k_sweep<{model}>" if a.observables else f"k_sweep_fast<{model}> (row kernel)"), 1
 
 
 def batched(a):
@@ -392,7 +410,7 @@ def batched(a):
         "config": {"workload": w["workload"], "walkers": w["walkers"], "sweeps_per_step": n,
                    "observables": a.observables},
         "roofline": {"bound": "lds", "achieved": achieved, "peak": peak, "unit": "GB/s",
-                     "frac": achieved / peak, "traffic": None, "kernel": w["kernel"],
+                     "frac": achieved / peak, "traffic": None, "kernel": sweep_kernel_of(a)[0],
                      "peak_source": "rewl_selfcheck(2)", "avg_launch_ms": avg_launch_s * 1e3,
                      "bytes_per_attempt": 32.5,
                      "hbm": {"peak": HBM_PEAK_GBS, "algorithmic_frac": achieved / HBM_PEAK_GBS}},
@@ -764,12 +782,12 @@ def config2_warm_leg(systems, params, a):
     return out
 
 
-def latency_model(cycles, clock_ghz, walkers, walkers_per_wave, default_launch):
+def latency_model(cycles, clock_ghz, walkers, sixteen):
     """Cycles per attempt per walker: the walker wavefront's chain is the bound
     of this workload."""
     out = {"cycles_per_attempt_per_walker": cycles, "clock_ghz_nominal": clock_ghz, "cus": 256}
-    if default_launch:
-        out.update({"walker_wavefronts": -(-walkers // walkers_per_wave), "walkers_per_wavefront": walkers_per_wave})
+    if sixteen:
+        out.update({"walker_wavefronts": -(-walkers // 4), "walkers_per_wavefront": 4})
     return out
 
 
@@ -838,12 +856,12 @@ def main():
     att_per_launch = attempts / max(launches, 1)
     achieved = att_per_launch * BYTES_PER_ATTEMPT / avg_launch_s / 1e9
     lnf = min(w["lnf"] for w in (eng.window_info(k) for k in range(eng.num_windows)))
-    default_launch = a.sweep_kernel == 0 and a.producers == 0 and a.walkers_per_group == 0 and not a.observables
-    traffic = MEASURED_TRAFFIC.get(params["sweeps_per_check"]) if default_launch else None
+    kernel, lanes = sweep_kernel_of(a)
+    sixteen = lanes == 16
+    traffic = MEASURED_TRAFFIC.get(params["sweeps_per_check"]) if sixteen and not a.observables else None
 
     peak = lds_peak()
     clock_ghz = 2.4
-    walkers_per_wave = 4
     cycles = avg_launch_s * clock_ghz * 1e9 / (att_per_launch / W)
     line = {
         "metric": "spin-flip attempts/s; time to ln f=1e-6 (learned warm start vs plain)",
@@ -865,7 +883,7 @@ def main():
             "sweeps_per_step": params["sweeps_per_check"],
             "sweeps_per_exchange": params["sweeps_per_exchange"],
             "attempts_per_step": attempts // a.steps,
-            "parallelism": ("sixteen lanes" if default_launch else "one lane") + " per walker, 1 GPU",
+            "parallelism": ("sixteen lanes" if sixteen else "one lane") + " per walker, 1 GPU",
             "producers": a.producers,
             "sweep_kernel": a.sweep_kernel,
             "observables": a.observables,
@@ -881,9 +899,7 @@ def main():
             "frac": achieved / peak,
             "traffic": traffic,
             "peak_source": "rewl_selfcheck(2): 16-byte conflict-free LDS reads on every CU of this GPU",
-            "kernel": "k_sweep_tree<Ising> (sixteen lanes per walker)" if default_launch
-                      else "k_sweep_tuned<Ising, L=64> (row-unrolled sweep)" if a.sweep_kernel in (0, 2, 3, 4)
-                      else "k_sweep_fast<Ising> (row kernel)",
+            "kernel": kernel,
             "avg_launch_ms": avg_launch_s * 1e3,
             "attempts_per_launch": att_per_launch,
             "bytes_per_attempt": BYTES_PER_ATTEMPT,
@@ -892,7 +908,7 @@ def main():
                     "frac": traffic / avg_launch_s / 1e9 / HBM_PEAK_GBS if traffic else None},
             # one walker is one sequential chain: what bounds this workload is
             # the walker wavefront's time per attempt, not a bandwidth
-            "latency": latency_model(cycles, clock_ghz, W, walkers_per_wave, default_launch),
+            "latency": latency_model(cycles, clock_ghz, W, sixteen),
         },
         "state": {"min_lnf_after": lnf, "flat_events": st1["flat_events"],
                   "exchanges_accepted": st1["exchanges_accepted"]},
