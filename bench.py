@@ -44,7 +44,7 @@ MPIEXEC = "/opt/conda/bin/mpiexec"
 # kernel, keyed by sweeps per launch: rocprofv3 --pmc FETCH_SIZE (x 2.0) and
 # WRITE_SIZE (x 1.0), the scales read off a plain 256 MiB copy
 # (profiles/k_sweep_tree_ising_L64_counters.md).
-MEASURED_TRAFFIC = {1000: (2.0 * 17504.89 + 1.0 * 8580.0) * 1024}
+MEASURED_TRAFFIC = {1000: (2.0 * 3606.375 + 1.0 * 6691.0) * 1024}
 
 
 def parse():

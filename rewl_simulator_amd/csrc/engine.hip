@@ -4,8 +4,9 @@
 // host builds the windows (glazier EQUAL_WINDOWS, glazier.hpp:69-115), packs
 // walkers into wavefront groups, uploads the tables, and then drives the
 // device with four kinds of launch that replace the reference's per-rank loop
-// and its MPI traffic: sweep (one lane per walker), exchange (one wavefront
-// per adjacent window pair), check (one wavefront per window) and finalize.
+// and its MPI traffic: sweep (sixteen lanes per walker, or one), exchange (up to
+// sixteen wavefronts per adjacent window pair), check (one wavefront per
+// window) and finalize.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 

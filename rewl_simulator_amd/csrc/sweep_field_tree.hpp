@@ -493,8 +493,8 @@ __device__ __forceinline__ void field_tree_terms(const DevGroup& G, const DevSys
     }
 }
 
-// One workgroup = one walker wavefront (four walkers) + two producers; groups
-// are taken persistently in blockIdx order.
+// One workgroup = one walker wavefront (four walkers) + two producers.  The grid
+// has one for every group of the list; the loop is for a smaller one.
 template <int MODEL>
 __global__ void __launch_bounds__(3 * kLanes, 3)
     k_sweep_field_tree(KArgs a, const int32_t* groups, int ngroups, int nsweeps, uint64_t sweep_base) {

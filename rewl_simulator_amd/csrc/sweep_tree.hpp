@@ -830,8 +830,8 @@ __device__ __forceinline__ void tree_fill(const DevGroup& G, const DevSystem& S,
     }
 }
 
-// One workgroup = one walker wavefront (four walkers) + one producer; groups
-// are taken persistently in blockIdx order.
+// One workgroup = one walker wavefront (four walkers) + one producer.  The grid has
+// one for every group of the list; the loop is for a smaller one.
 template <int MODEL, int OBS>
 __global__ void __launch_bounds__(2 * kLanes) k_sweep_tree(KArgs a, const TreeScale* scale, const int32_t* groups,
                                                            int ngroups, int nsweeps, uint64_t sweep_base) {
